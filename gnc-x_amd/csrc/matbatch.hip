@@ -27,8 +27,8 @@
 // with each block's scale, so a block's integer dot is exact in one (Q6_K:
 // two) products per K slice; the block scale is applied on the VALU and d
 // and the min term once per super-block.
-// BF16 weights (fp32 activations, cpp:1432-1461) use the slot-dot kernel: a
-// wave per (row, token).
+// BF16 weights (fp32 activations, cpp:1432-1461): matbatch_bf16_kernel, the
+// activations as three exact bf16 parts.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -45,27 +45,23 @@ using namespace dev;
 
 constexpr int kThreads = 256;
 
-template <int TYPE>
+// BF16 products of little work: one wave per (row, token)
 __global__ __launch_bounds__(kThreads) void matbatch_rowtok_kernel(const uint8_t* __restrict w, size_t rbytes,
-                                                                   const float* __restrict x,
-                                                                   const int8_t* __restrict q,
-                                                                   const ActMeta* __restrict meta, int32_t k,
-                                                                   int32_t n, float* __restrict y) {
+                                                                   const float* __restrict x, int32_t k, int32_t n,
+                                                                   float* __restrict y) {
     const int lane = threadIdx.x & 63;
     const int32_t r = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
     const int32_t t = blockIdx.y;
     if (r >= n) return;
     const uint8_t* row = w + static_cast<size_t>(r) * rbytes;
-    const int8_t* qt = q + static_cast<size_t>(t) * k;
-    const ActMeta* mt = meta + static_cast<size_t>(t) * (k / 32);
-    using S = Slot<TYPE>;
+    using S = Slot<kBF16>;
     const int32_t slots = S::slots(k);
     float acc = 0.0f;
     for (int32_t s = lane; s < slots; s += 64) {
         typename S::Frag f;
         typename S::Act a;
         S::load(f, PtrRow{row}, s);
-        slot_act<TYPE>(a, s, qt, mt, x + static_cast<size_t>(t) * k);
+        slot_act<kBF16>(a, s, nullptr, nullptr, x + static_cast<size_t>(t) * k);
         acc += S::dot(f, a, s);
     }
     acc = wave_sum(acc);
@@ -1287,6 +1283,261 @@ __global__ __launch_bounds__(64 * RT, 1) void matbatch_qs_stream_kernel(
     }
 }
 
+// ---- BF16 weights, fp32 activations -------------------------------------------
+//
+// The reference multiplies fp32 activations with BF16 weights in fp32
+// (cpp:1432-1461).  Here the product runs on the bf16 matrix cores without
+// rounding the activations: x = h + m + l exactly, each part the top 16 bits
+// of what the parts before it left (8 significant bits each, 24 in all), and
+// three v_mfma_f32_16x16x32_bf16 per tile and 32-value K slice.  Every
+// product of two bf16 values is exact in fp32.
+//
+// A work-group is 8 waves of MT 16-row weight fragments each (128 MT rows)
+// times 16 NT tokens.  A weight operand is 16 bytes of one row, so the waves
+// load theirs from memory straight into registers, a stage (128 of K) ahead;
+// the tokens' fp32 values are loaded a stage ahead too, split on their way
+// into LDS (three bf16 arrays per stage, two stages) and read from there by
+// every wave.  Each stage is a sum of its own, the smaller parts first; eight
+// stages add up in T and those sums in acc, so no chain of roundings at the
+// full size is longer than K / 1024.  Against the 64-bit product (relative L2)
+// at K = 256 / 1024 / 4096 / 14336: 0.70 / 0.80 / 0.93-1.05 / 1.07-1.28e-7;
+// matbatch_rowtok_kernel 0.87 / 0.94 / 1.06 / 1.35e-7; one chain over all
+// stages, folded every 256 values, 1.3-1.7e-7.
+// Bound: the weight bytes up to about 64 tokens, then the three products (960
+// of the 1114 bf16 TFLOP/s a large library product reaches here at 4096 x
+// 4096, B = 2048).
+constexpr int kBfKs = 128;  // K per stage
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// bf16 parts of 8 values: truncated top 16 bits, the remainder again, and the
+// rest (exact: at most 8 significant bits are left).  Infinite or NaN values
+// leave NaN in the lower parts (the epilogue's check).
+__device__ __forceinline__ void split3(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
+    uint32_t ho[4], mo[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t p[3][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float a = v[2 * i + e];
+            p[0][e] = __builtin_bit_cast(uint32_t, a);
+            const float r1 = a - __builtin_bit_cast(float, p[0][e] & 0xffff0000u);
+            p[1][e] = __builtin_bit_cast(uint32_t, r1);
+            const float r2 = r1 - __builtin_bit_cast(float, p[1][e] & 0xffff0000u);
+            p[2][e] = __builtin_bit_cast(uint32_t, r2);
+        }
+        ho[i] = __builtin_amdgcn_perm(p[0][1], p[0][0], 0x07060302u);
+        mo[i] = __builtin_amdgcn_perm(p[1][1], p[1][0], 0x07060302u);
+        lo[i] = __builtin_amdgcn_perm(p[2][1], p[2][0], 0x07060302u);
+    }
+    h = make_uint4(ho[0], ho[1], ho[2], ho[3]);
+    m = make_uint4(mo[0], mo[1], mo[2], mo[3]);
+    l = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+}
+
+template <int MT, int NT>
+__global__ __launch_bounds__(512, 1) void matbatch_bf16_kernel(const uint8_t* __restrict w, size_t rbytes,
+                                                               const float* __restrict x, int32_t b, int32_t k,
+                                                               int32_t n, int32_t kchunk, float* __restrict y,
+                                                               float* __restrict part, int32_t xmap_tg) {
+    constexpr int WR = 16 * MT, BN = 8 * WR, BM = 16 * NT;  // rows per wave and group, tokens
+    constexpr int KS = kBfKs, NKS = KS / 32, SEGS = KS / 8;
+    constexpr int XI = BM * SEGS >= 512 ? BM * SEGS / 512 : 1;  // 8-value pieces per thread and stage
+    constexpr int OLD = BN + 4;                                 // floats per output row in LDS
+    constexpr size_t kXBytes = size_t{2} * 3 * BM * KS * 2, kOBytes = size_t{4} * BM * OLD;
+    __shared__ __align__(16) char smem[kXBytes > kOBytes ? kXBytes : kOBytes];
+    // part p of stage s: [token][KS] with the 16-byte segments of token t at
+    // positions c ^ (t % 16), so 16 tokens reading one segment hit distinct banks
+    auto xs = [&](int s, int p) { return reinterpret_cast<uint16_t*>(smem) + (s * 3 + p) * BM * KS; };
+
+    int bx, by, bz;
+    if (xmap_tg > 0) {  // token groups dealt over the XCDs (as matbatch_qs_stream_kernel)
+        const int lin = static_cast<int>(blockIdx.x), xcd = lin & 7, slot = lin >> 3, tpx = xmap_tg / 8;
+        bx = slot / tpx;
+        by = xcd * tpx + slot % tpx;
+        bz = 0;
+    } else if (xmap_tg < 0) {  // row groups
+        const int lin = static_cast<int>(blockIdx.x), xcd = lin & 7, slot = lin >> 3;
+        const int rgs = -xmap_tg, tgs = static_cast<int>(gridDim.x) / rgs;
+        bx = xcd * (rgs / 8) + slot / tgs;
+        by = slot % tgs;
+        bz = 0;
+    } else {
+        bx = static_cast<int>(blockIdx.x);
+        by = static_cast<int>(blockIdx.y);
+        bz = static_cast<int>(blockIdx.z);
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const int32_t t0 = by * BM, n0 = bx * BN;
+    const int32_t kb = bz * kchunk, ke = min(k, kb + kchunk);
+    const int32_t nst = (ke - kb + KS - 1) / KS;
+    const int32_t rows_here = min(BM, b - t0), wrows_here = min(BN, n - n0);
+
+    // rows past N, tokens past B and values past the range read zeros
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(w + static_cast<size_t>(n0) * rbytes), static_cast<short>(0),
+        wrows_here * static_cast<int32_t>(rbytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(x + static_cast<size_t>(t0) * k), static_cast<short>(0),
+        rows_here * k * static_cast<int32_t>(sizeof(float)), 0x00020000);
+    u32x4 wr[2][NKS][MT], xr[XI][2];
+    auto wload = [&](u32x4 (&r)[NKS][MT], int32_t s) {
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const int32_t kp = kb + s * KS + 32 * ks + 8 * lg;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int32_t row = wv * WR + 16 * i + l16;
+                const int32_t off = kp < ke ? row * static_cast<int32_t>(rbytes) + 2 * kp : kMfOob;
+                r[ks][i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, row < wrows_here ? off : kMfOob, 0, 0);
+            }
+        }
+    };
+    auto xload = [&](int32_t s) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int32_t t = (tid + 512 * i) / SEGS, kp = kb + s * KS + 8 * (tid % SEGS);
+            const int32_t off = t < rows_here && kp < ke ? (t * k + kp) * static_cast<int32_t>(sizeof(float)) : kMfOob;
+            xr[i][0] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
+            xr[i][1] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 16, 0);
+        }
+    };
+    auto xstore = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int t = (tid + 512 * i) / SEGS, c = (tid % SEGS) ^ (t & 15);
+            if (BM * SEGS < 512 && t >= BM) continue;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const u32x4 q = xr[i][e >> 2];
+                v[e] = __builtin_bit_cast(float, (e & 3) == 0 ? q.x : (e & 3) == 1 ? q.y : (e & 3) == 2 ? q.z : q.w);
+            }
+            uint4 h, m, l;
+            split3(v, h, m, l);
+            *reinterpret_cast<uint4*>(xs(s, 0) + t * KS + 8 * c) = h;
+            *reinterpret_cast<uint4*>(xs(s, 1) + t * KS + 8 * c) = m;
+            *reinterpret_cast<uint4*>(xs(s, 2) + t * KS + 8 * c) = l;
+        }
+    };
+    floatx4 acc[MT][NT], T[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = T[i][j] = floatx4{};
+    auto compute = [&](const u32x4 (&r)[NKS][MT], int s) {
+        floatx4 S[MT][NT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) S[i][j] = floatx4{};
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+            const uint16_t* xp = xs(s, p);
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                bf16x8 xo[NT];
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    xo[j] = *reinterpret_cast<const bf16x8*>(xp + (16 * j + l16) * KS + 8 * ((4 * ks + lg) ^ l16));
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        S[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, r[ks][i]), xo[j],
+                                                                         S[i][j], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) T[i][j][e] += S[i][j][e];
+    };
+    auto fold = [&] {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc[i][j][e] += T[i][j][e];
+                    T[i][j][e] = 0.0f;
+                }
+    };
+
+    // stage s from register set and LDS stage s % 2: the next stage's loads
+    // are issued first (x before the weights: the wait for x then leaves the
+    // weights in flight), its x goes to the other LDS stage, and the barrier
+    // makes it visible (step_barrier waits for no loads here)
+    xload(0);
+    wload(wr[0], 0);
+    xstore(0);
+    step_barrier<63>();
+    for (int32_t s = 0; s < nst; s += 2) {
+        xload(s + 1);
+        wload(wr[1], s + 1);
+        compute(wr[0], 0);
+        if (s + 1 >= nst) break;
+        xstore(1);
+        step_barrier<63>();
+        xload(s + 2);
+        wload(wr[0], s + 2);
+        compute(wr[1], 1);
+        if ((s & 7) == 6) fold();
+        xstore(0);
+        step_barrier<63>();
+    }
+    fold();
+
+    // Infinite and NaN inputs: the parts of an infinite x and the products of
+    // zero parts with an infinite weight are NaN where the fp32 product need
+    // not be; an output that came out NaN is formed again in plain fp32
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int32_t r = wv * WR + 16 * i + 4 * lg + e, t = 16 * j + l16;
+                if (acc[i][j][e] != acc[i][j][e] && r < wrows_here && t < rows_here) {
+                    const uint16_t* wp = reinterpret_cast<const uint16_t*>(w + static_cast<size_t>(n0 + r) * rbytes);
+                    const float* xp = x + static_cast<size_t>(t0 + t) * k;
+                    float sum = 0.0f;
+                    for (int32_t q = kb; q < ke; ++q)
+                        sum += __builtin_bit_cast(float, static_cast<uint32_t>(wp[q]) << 16) * xp[q];
+                    acc[i][j][e] = sum;
+                }
+            }
+
+    // the tile through LDS as [token][row], then whole token rows out
+    __syncthreads();
+    float* ost = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            *reinterpret_cast<floatx4*>(&ost[(16 * j + l16) * OLD + wv * WR + 16 * i + 4 * lg]) = acc[i][j];
+    __syncthreads();
+    float* dst = gridDim.z > 1 ? part + static_cast<size_t>(bz) * b * n : y;
+    if ((n & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+        constexpr int LPT = BN / 4, TPI = 512 / LPT;
+        const int c = 4 * (tid % LPT);
+        for (int t = tid / LPT; t < rows_here; t += TPI)
+            if (c < wrows_here)
+                *reinterpret_cast<floatx4*>(&dst[static_cast<size_t>(t0 + t) * n + n0 + c]) =
+                    *reinterpret_cast<const floatx4*>(&ost[t * OLD + c]);
+    } else {
+        for (int e = tid; e < rows_here * BN; e += 512) {
+            const int t = e / BN, c = e % BN;
+            if (c < wrows_here) dst[static_cast<size_t>(t0 + t) * n + n0 + c] = ost[t * OLD + c];
+        }
+    }
+}
+
 // y = sum over the split K ranges, added in range order (deterministic);
 // range z's partials are the flat block [z count, (z + 1) count).  The
 // first kRedU ranges are loaded together before the adds (a loop of
@@ -1422,6 +1673,17 @@ struct Q4kPlan {
     int32_t xmap = 0;  // token groups of the XCD-aware order (> 0), minus row groups (< 0), 0: grid order
 };
 
+// The XCD order of rg x tg work-groups with the least L2-miss traffic,
+// counting each XCD's own reads of w weight and x activation bytes: by token
+// groups (> 0) every XCD reads all weights and its share of the activations;
+// by row groups (< 0) one XCD reads each weight and every XCD the activations
+// once per round of 32 work-groups (rg tg / 256).  0: grid order.
+int32_t xcd_order(int64_t rg, int64_t tg, double w, double x) {
+    const double by_tok = 8.0 * w + x, by_row = w + 8.0 * x * std::max(1.0, static_cast<double>(rg * tg) / 256.0);
+    if (rg % 8 == 0 && (tg % 8 != 0 || by_row < by_tok)) return -static_cast<int32_t>(rg);
+    return tg % 8 == 0 ? static_cast<int32_t>(tg) : 0;
+}
+
 // Row groups of 256 x 64 tokens, K split in ranges of whole super-blocks
 // until about 256 work-groups run (one per CU).
 Q4kPlan q4k_stream_plan(int32_t b, int32_t k, int32_t n) {
@@ -1433,17 +1695,9 @@ Q4kPlan q4k_stream_plan(int32_t b, int32_t k, int32_t n) {
     const int32_t csb = (nsb + splits - 1) / splits;
     p.kchunk = csb * 256;
     p.splits = (nsb + csb - 1) / csb;
-    // the XCD order with the least L2-miss traffic, counting each XCD's own
-    // reads: by token groups every XCD reads all weights W and its share of
-    // the activations X; by row groups one XCD reads each weight and every
-    // XCD the activations once per round of 32 work-groups (rg tg / 256)
     p.xmap = 0;
-    if (p.splits == 1) {
-        const double w = static_cast<double>(n) * (k / 256) * 210.0, x = static_cast<double>(b) * k * 2.2;
-        const double by_tok = 8.0 * w + x, by_row = w + 8.0 * x * std::max(1.0, static_cast<double>(wgs) / 256.0);
-        if (rg % 8 == 0 && (tg % 8 != 0 || by_row < by_tok)) p.xmap = -static_cast<int32_t>(rg);
-        else if (tg % 8 == 0) p.xmap = static_cast<int32_t>(tg);
-    }
+    if (p.splits == 1)
+        p.xmap = xcd_order(rg, tg, static_cast<double>(n) * (k / 256) * 210.0, static_cast<double>(b) * k * 2.2);
     return p;
 }
 
@@ -1538,17 +1792,63 @@ hipError_t launch_q4k(const uint8_t* w, const float* x, int32_t b, int32_t k, in
     return launch_q4k_mats(m, xhl, pq, rscale, b, k, p, part, stream);
 }
 
-template <int TYPE>
-hipError_t launch_t(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, int8_t* q,
-                    ActMeta* meta, hipStream_t stream) {
-    if (TYPE != kBF16) {
-        hipError_t e = launch_act_quant(x, b, k, q, meta, stream);
-        if (e != hipSuccess) return e;
-    }
-    dim3 grid((n + 3) / 4, b);
-    hipLaunchKernelGGL(matbatch_rowtok_kernel<TYPE>, grid, dim3(kThreads), 0, stream, w, row_bytes(TYPE, k), x, q,
-                       meta, k, n, y);
+// BF16: 256 rows per row group and 16, 32 or 64 tokens, K split in ranges of
+// whole 256-value pairs of stages until about 256 work-groups run.
+// Measured at 4096 x 4096, B = 64 / 100 / 512: 20.7 / 23.8 / 61.8 us; with
+// about 128 work-groups 20.9 / 31.1 / 89.5, with 128 rows per row group 17.9 /
+// 24.7 / 66.3 (but 50.2 against 44.5 us at 4096 x 14336, B = 64).
+constexpr int kBfMT = 2;
+struct BfPlan {
+    int nt;
+    int32_t splits, kchunk, xmap;
+};
+BfPlan bf16_plan(int32_t b, int32_t k, int32_t n) {
+    BfPlan p{b <= 16 ? 1 : b <= 32 ? 2 : 4, 1, k, 0};
+    const int32_t units = (k + 255) / 256;
+    const int64_t rg = (n + 128 * kBfMT - 1) / (128 * kBfMT), tg = (b + 16 * p.nt - 1) / (16 * p.nt), wgs = rg * tg;
+    int32_t splits = wgs >= 256 ? 1 : static_cast<int32_t>(256 / wgs);
+    splits = std::max(1, std::min(splits, units));
+    const int32_t per = (units + splits - 1) / splits;
+    p.kchunk = per * 256;
+    p.splits = (units + per - 1) / per;
+    if (p.splits == 1) p.xmap = xcd_order(rg, tg, static_cast<double>(n) * k * 2.0, static_cast<double>(b) * k * 4.0);
+    return p;
+}
+
+// The matrix kernel's fixed cost (one or two launches of long-lived
+// work-groups, K split) against a wave per output: up to 4 10^7 products the
+// latter.  Measured rowtok / matrix kernel: 1024 x 512 at B = 48 / 100: 6.6 /
+// 12.8 and 11.7 / 13.0 us; 4096 x 4096 at B = 2 / 5: 8.4 / 11.3 and 17.2 /
+// 11.3 us; 14336 x 4096 at B = 2: 38.0 / 29.0 us.
+bool bf16_small(int32_t b, int32_t k, int32_t n) { return static_cast<double>(b) * k * n <= 4.0e7; }
+
+template <int NT>
+hipError_t launch_bf16_t(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, float* part,
+                         const BfPlan& p, hipStream_t stream) {
+    const int32_t rg = (n + 128 * kBfMT - 1) / (128 * kBfMT), tg = (b + 16 * NT - 1) / (16 * NT);
+    const dim3 grid = p.xmap != 0 ? dim3(rg * tg) : dim3(rg, tg, p.splits);
+    hipLaunchKernelGGL((matbatch_bf16_kernel<kBfMT, NT>), grid, dim3(512), 0, stream, w, row_bytes(kBF16, k), x, b, k, n,
+                       p.kchunk, y, part, p.xmap);
     return hipGetLastError();
+}
+
+hipError_t launch_bf16(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, float* part,
+                       hipStream_t stream) {
+    if (bf16_small(b, k, n)) {
+        hipLaunchKernelGGL(matbatch_rowtok_kernel, dim3((n + 3) / 4, b), dim3(kThreads), 0, stream, w,
+                           row_bytes(kBF16, k), x, k, n, y);
+        return hipGetLastError();
+    }
+    const BfPlan p = bf16_plan(b, k, n);
+    const hipError_t e = p.nt == 1   ? launch_bf16_t<1>(w, x, b, k, n, y, part, p, stream)
+                         : p.nt == 2 ? launch_bf16_t<2>(w, x, b, k, n, y, part, p, stream)
+                                     : launch_bf16_t<4>(w, x, b, k, n, y, part, p, stream);
+    if (e != hipSuccess || p.splits == 1) return e;
+    RedMats r{};
+    r.y[0] = y;
+    r.end[0] = static_cast<size_t>(b) * n;
+    r.count = 1;
+    return launch_reduce(part, p.splits, r, stream);
 }
 
 }  // namespace
@@ -1568,7 +1868,10 @@ static size_t pq_bytes(int32_t type, int32_t b, int32_t k) {
 }
 
 size_t matbatch_workspace_bytes(int32_t type, int32_t b, int32_t k, int32_t n) {
-    if (type == kBF16) return 256;
+    if (type == kBF16) {
+        const int32_t splits = bf16_small(b, k, n) ? 1 : bf16_plan(b, k, n).splits;
+        return (splits > 1 ? static_cast<size_t>(splits) * b * n * sizeof(float) : 0) + 256;
+    }
     const int32_t splits = type == kQ4_K                     ? q4k_plan(b, k, n).splits
                            : type == kQ6_K && GNCX_Q6K_STREAM ? q4k_stream_plan(b, k, n).splits
                                                               : mfma_plan(b, k, n).splits;
@@ -1603,7 +1906,7 @@ hipError_t launch_matbatch(int32_t type, const uint8_t* w, const float* x, int32
     case kQ6_K:
         return GNCX_Q6K_STREAM ? launch_q6ks(w, x, b, k, n, y, xhl, rscale, part, stream, up)
                                : launch_mfma<kQ6_K>(w, x, b, k, n, y, xhl, rscale, part, stream, up);
-    case kBF16: return up ? hipErrorNotSupported : launch_t<kBF16>(w, x, b, k, n, y, nullptr, nullptr, stream);
+    case kBF16: return up ? hipErrorNotSupported : launch_bf16(w, x, b, k, n, y, static_cast<float*>(workspace), stream);
     default: return hipErrorInvalidValue;
     }
 }

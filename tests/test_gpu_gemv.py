@@ -277,6 +277,57 @@ def test_matbatch_parity(lib, oracle, t, k, n, b):
     assert err < (TOL if t == BF16 else TOL_MATBATCH)
 
 
+# BF16 weights on the bf16 matrix cores, the fp32 activations as three exact
+# bf16 parts (from 4e7 products; one small case below it): K past one and two 128-value stages and past
+# the 1024-value fold, ragged rows and tokens around the 16 / 32 / 64-token
+# tiles, K split and unsplit.  Every product is exact; an output is a sum of
+# 3 K products with at most 3 * 4 + 8 + K / 1024 + 256 roundings on its way
+# (stage, eight stages, folds, K ranges), each at most 2^-23 (the matrix
+# cores may truncate) of sum |w x|.
+@pytest.mark.parametrize("k,n,b", [(8, 1, 1), (136, 8200, 40), (264, 9003, 17), (4096, 700, 16), (1032, 1000, 64),
+                                   (2048, 1001, 130), (256, 16500, 300), (14336, 1500, 2)])
+def test_matbatch_bf16_exact_parts(lib, k, n, b):
+    w = synth.make_weights(BF16, n, k, seed=8300 + k + n)
+    x = (synth.make_activations(b, k, seed=8400 + k + b).reshape(b, k) * np.float32(3.0)).astype(np.float32)
+    y = np.full((b, n), np.nan, np.float32)
+    lib.gncx_xfold_universal_matbatch(ptr(w), 0, BF16, ptr(x), b, k, n, ptr(y), None)
+    gncx.check(lib)
+    wf = (w.view(np.uint16).astype(np.uint32) << 16).view(np.float32).reshape(n, k).astype(np.float64)
+    err = np.abs(y - x.astype(np.float64) @ wf.T)
+    roundings = 3 * 4 + 8 + k // 1024 + 256
+    assert np.all(err <= roundings * 2.0 ** -23 * (np.abs(x.astype(np.float64)) @ np.abs(wf).T) + 1e-37)
+    assert rel_l2(y, x.astype(np.float64) @ wf.T) < 3e-7  # measured 0.7e-7 to 1.3e-7
+
+
+def test_matbatch_bf16_infinite_and_nan(lib):
+    """Infinite and NaN activations and weights give what the fp32 products
+    give: a zero lower part times an infinite weight is no NaN."""
+    k, n, b = 2048, 1000, 40
+    w = synth.make_weights(BF16, n, k, seed=8500)
+    x = synth.make_activations(b, k, seed=8501).reshape(b, k).copy()
+    x[0, 5] = np.inf
+    x[1, 7] = -np.inf
+    x[2, 9] = np.nan
+    x[3, 11] = 0.0
+    # near the top of fp32 in one place: |w| < 0.2 there, so no sum in any order
+    # leaves fp32 (a whole row of such values overflows in some orders only)
+    x[4, 3] = np.float32(3.4e38)
+    wu = w.view(np.uint16).reshape(n, k)
+    wu[10, 11] = 0x7F80  # +inf
+    wu[11, 12] = 0xFF80  # -inf
+    y = np.zeros((b, n), np.float32)
+    lib.gncx_xfold_universal_matbatch(ptr(w), 0, BF16, ptr(x), b, k, n, ptr(y), None)
+    gncx.check(lib)
+    wf = (wu.astype(np.uint32) << 16).view(np.float32)
+    with np.errstate(all="ignore"):
+        want = np.stack([(x[t][None, :] * wf).astype(np.float64).sum(1) for t in range(b)])
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    big = np.abs(want) > 3e38
+    assert np.array_equal(np.sign(y[big]), np.sign(want[big]))
+    inf = np.isinf(want)
+    assert np.array_equal(y[inf], want[inf].astype(np.float32))
+
+
 # Q6_K scales beyond +-64 (real quantisers use the whole int8 range): then
 # sc (q - 32) can exceed 2048 and the 256-token tiles add the third product in
 # the steps that hold such a scale.  All rows large, none, and one row in
