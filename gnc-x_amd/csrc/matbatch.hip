@@ -6,32 +6,23 @@
 // same integer block dot as the matvec; the output is row-major out[t*N + m].
 //
 // Quantised weights (Q4_0, Q8_0, Q4_K, Q6_K) go through the fp16 matrix
-// cores with both operands carried as fp16 pairs (hi, lo):
-//   1. act_hilo_kernel quantises each token row exactly as the reference
-//      does and stores each quantised activation q * d / s as an fp16 pair
-//      (s is a power-of-two row scale the MFMA epilogue multiplies back),
-//   2. matbatch_mfma_kernel streams 32-wide K steps: the work-group's weight
-//      rows are dequantised block by block in fp32 and split into fp16 pairs
-//      in LDS, its token rows are copied into LDS, and each wave runs three
-//      v_mfma_f32_32x32x16_f16 per tile and K slice (hi x hi, lo x hi,
-//      hi x lo) with fp32 accumulation.
-// Each product is then exact to about 2^-22, and Y lands within about 2e-7
-// relative L2 of the reference's integer block dots (fp16 operands alone:
-// 3e-4).  An int8 MFMA path would be exact too, but its per-32-block scales
-// cost ~3 VALU operations per output and block, several times the
-// matrix-core time of the three fp16 products.
-// Q4_K (the layer format of the prefill workloads) and Q6_K have their own
-// kernel, matbatch_qs_stream_kernel: the weights are small integers exact in
-// fp16 (sc q; sc (q - 32) as two parts) with d (and dmin) fixed per
-// 256-value super-block, and the activations are the quantised q as fp16
-// with each block's scale, so a block's integer dot is exact in one (Q6_K:
-// two) products per K slice; the block scale is applied on the VALU and d
-// and the min term once per super-block.
+// cores with exact integer operands:
+//   1. act_q_kernel quantises each token row exactly as the reference does
+//      and stores the quantised q as fp16 with each block's scale (and
+//      launch_norm_act_q does so for the RMSNorm of a row);
+//   2. matbatch_qs_stream_kernel streams the weights through registers; each
+//      32-value block of a tile is one exact integer dot (Q6_K: two) on the
+//      matrix cores, and the block scales are applied in fp32 on the VALU.
+// Y lands within about 1e-7 relative L2 of the reference's integer block
+// dots.  An int8 MFMA path would be exact too, but adds a conversion per
+// output and block to that VALU work, which is what bounds the kernel.
 // BF16 weights (fp32 activations, cpp:1432-1461): matbatch_bf16_kernel, the
 // activations as three exact bf16 parts.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "gncx_act.h"
 #include "gncx_device.h"
@@ -72,49 +63,31 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2 __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// fp16 pair (hi, lo) of a float: hi = fp16(v) and lo = fp16(v - hi), with
-// v - hi exact in fp32, so hi + lo carries 22 significant bits of v.
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-    const _Float16 ha = static_cast<_Float16>(a), hb = static_cast<_Float16>(b);
-    const _Float16 la = static_cast<_Float16>(a - static_cast<float>(ha));
-    const _Float16 lb = static_cast<_Float16>(b - static_cast<float>(hb));
-    hi = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, ha)) |
-         (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, hb)) << 16);
-    lo = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, la)) |
-         (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, lb)) << 16);
-}
-
-// act_hilo_kernel<U> holds U float4 of x per thread in registers from the
+// act_q_kernel<U> holds U float4 of x per thread in registers from the
 // max pass to the quantising pass (rows up to 4 kThreads U values): the
 // loads of a row are issued together, and a longer row reads its tail again.
-// U = 4 covers 4096-wide rows at 40-odd registers; wider rows take U = 16
-// (130-odd registers, 3 waves per SIMD), or, for the SwiGLU rows of the down
-// projection up to 12288 wide, 1024 threads (NT) with U = 3, which keeps more
-// of a row's loads in flight (47.9 -> 45.1 us at 2048 x 12288).
+// U = 4 covers 4096-wide rows; wider rows take U = 16, or, for the SwiGLU rows
+// of the down projection up to 12288 wide, 1024 threads (NT) with U = 3, which
+// keeps more of a row's loads in flight (47.9 -> 45.1 us at 2048 x 12288).
 
-// The reference's per-32 quantisation of row blockIdx.x of x (cpp:955-995),
-// each quantised value a = q * d (one fp32 rounding) scaled by 1 / s, where
-// s is the power of two above the row's largest |x| (stored in rscale; the
-// MFMA epilogue multiplies it back, exactly), and stored as its fp16 pair
-// (hi, lo): xhl holds, per 8 elements, 16 bytes of hi then 16 bytes of lo.
-// The rescale keeps every value in [-1, 1], so activations far beyond fp16's
-// range (SwiGLU outputs of 1e5 and more) keep the pair's relative precision.
+// The reference's per-32 quantisation of row blockIdx.x of x (cpp:955-995):
+// the quantised values q as fp16 (integers of at most 127, exact), row-major
+// [B x K], and each 32-block's d / s as fp32 [B x K / 32], s the power of two
+// above the row's largest |x| (stored in rscale; the product's epilogue
+// multiplies it back, exactly).  Within each 8 values the order is 0 2 1 3 4
+// 6 5 7, the product kernel's operand order.  With pq given (K a multiple of
+// 256), also each 32-block's sum of the quantised activations, P = (sum q) *
+// d / s, as an fp16 pair: per token row and 256-value super-block, 8 hi then
+// 8 lo values (the Q4_K kernel's min term, cpp:1177-1178); the scale keeps P
+// within fp16's range for activations of 1e5 and more (SwiGLU outputs).
 // One work-group per row: the row maximum first, then 8 lanes per 32-block,
 // 4 values per lane.
-// With pq given (K a multiple of 256), also each 32-block's sum of the
-// quantised activations, P = (sum q) * d / s, as an fp16 pair: per token row
-// and 256-value super-block, 8 hi then 8 lo values (the Q4_K kernel's min
-// term, cpp:1177-1178).
 // With SW the row is the SwiGLU of two rows, x the gates and up the ups
 // (the values gncx_swiglu_activation writes), formed as they are read.
-// With QX (the streamed Q4_K and Q6_K kernel) the quantised values q themselves
-// go out instead of the pairs, as fp16 (integers of at most 127, exact):
-// xhl holds 4 of them per task, row-major [B x K], and dxs (set) each
-// 32-block's d / s as fp32 [B x K / 32]; P as above.
-// One task's QX outputs (4 values of row `row`, task t of k / 4, at the
+// One task's outputs (4 values of row `row`, task t of k / 4, at the
 // row's 1 / s = inv): q as fp16, the block's d / s from its first lane and,
 // with pq, the block's P pair.  Whole 8-lane groups call it together.
-__device__ __forceinline__ void emit_qx(const float4 v, int32_t t, int32_t row, int32_t k, float inv,
+__device__ __forceinline__ void emit_q(const float4 v, int32_t t, int32_t row, int32_t k, float inv,
                                         uint2* __restrict xq, float* __restrict dxs, _Float16* __restrict pq) {
     const int32_t tasks = k / 4;
     int q0, q1, q2, q3;
@@ -124,7 +97,7 @@ __device__ __forceinline__ void emit_qx(const float4 v, int32_t t, int32_t row, 
         return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(a))) |
                (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(b))) << 16);
     };
-    xq[static_cast<size_t>(row) * tasks + t] = make_uint2(h2(q0, q1), h2(q2, q3));
+    xq[static_cast<size_t>(row) * tasks + t] = make_uint2(h2(q0, q2), h2(q1, q3));
     if ((t & 7) == 0) dxs[static_cast<size_t>(row) * (k / 32) + (t >> 3)] = d * inv;
     if (pq) {
         // the 8 lanes of block t / 8: quad sums, then lane i adds lane 7 - i
@@ -142,11 +115,10 @@ __device__ __forceinline__ void emit_qx(const float4 v, int32_t t, int32_t row, 
     }
 }
 
-template <int kHiloU, bool SW = false, bool QX = false, int NT = kThreads>
-__global__ __launch_bounds__(NT) void act_hilo_kernel(const float* __restrict x, int32_t k,
-                                                            uint2* __restrict xhl, float* __restrict rscale,
-                                                            _Float16* __restrict pq, const float* __restrict up,
-                                                            float* __restrict dxs = nullptr) {
+template <int U, bool SW = false, int NT = kThreads>
+__global__ __launch_bounds__(NT) void act_q_kernel(const float* __restrict x, int32_t k, uint2* __restrict xq,
+                                                   float* __restrict rscale, _Float16* __restrict pq,
+                                                   const float* __restrict up, float* __restrict dxs) {
     __shared__ float red[NT / 64];
     const int32_t row = blockIdx.x, tasks = k / 4;
     const float4* xg = reinterpret_cast<const float4*>(x + static_cast<size_t>(row) * k);
@@ -166,16 +138,16 @@ __global__ __launch_bounds__(NT) void act_hilo_kernel(const float* __restrict x,
     };
     const Row xr{xg, xu};
     auto amax4 = [](const float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
-    float4 xv[kHiloU];
+    float4 xv[U];
 #pragma unroll
-    for (int u = 0; u < kHiloU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int32_t t = static_cast<int32_t>(threadIdx.x) + u * NT;
         xv[u] = t < tasks ? xr[t] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     float m = 0.0f;
 #pragma unroll
-    for (int u = 0; u < kHiloU; ++u) m = fmaxf(m, amax4(xv[u]));
-    for (int32_t t = threadIdx.x + kHiloU * NT; t < tasks; t += NT) m = fmaxf(m, amax4(xr[t]));
+    for (int u = 0; u < U; ++u) m = fmaxf(m, amax4(xv[u]));
+    for (int32_t t = threadIdx.x + U * NT; t < tasks; t += NT) m = fmaxf(m, amax4(xr[t]));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -186,68 +158,55 @@ __global__ __launch_bounds__(NT) void act_hilo_kernel(const float* __restrict x,
     const float sc = m > 0.0f && m <= 3.0e38f ? ldexpf(1.0f, ilogbf(m) + 1) : 1.0f;  // power of two > m
     const float inv = 1.0f / sc;                                       // exact
     if (threadIdx.x == 0) rscale[row] = sc;
-    uint2* out = xhl + static_cast<size_t>(row) * tasks * 2;
-    auto emit = [&](const float4 v, int32_t t) {
-        if constexpr (QX) {
-            emit_qx(v, t, row, k, inv, xhl, dxs, pq);
-        } else {
-            int q0, q1, q2, q3;
-            float d;
-            quantize_values(v, q0, q1, q2, q3, d);
-            uint2 hi, lo;
-            split2((static_cast<float>(q0) * d) * inv, (static_cast<float>(q1) * d) * inv, hi.x, lo.x);
-            split2((static_cast<float>(q2) * d) * inv, (static_cast<float>(q3) * d) * inv, hi.y, lo.y);
-            // task t is elements 4t .. 4t + 3: chunk t / 2 of 8, half t % 2
-            uint2* c = out + 4 * (t >> 1) + (t & 1);
-            c[0] = hi;
-            c[2] = lo;
-            if (pq) {
-                // the 8 lanes of block t / 8: quad sums, then lane i adds lane 7 - i
-                const int s4 = quad_sum(q0 + q1 + q2 + q3);
-                const int sum = s4 + __builtin_amdgcn_mov_dpp(s4, 0x141, 0xf, 0xf, false);
-                if ((t & 7) == 0) {
-                    const int32_t blk = t >> 3;
-                    const float pv = (static_cast<float>(sum) * d) * inv;
-                    const _Float16 ph = static_cast<_Float16>(pv);
-                    const _Float16 pl = static_cast<_Float16>(pv - static_cast<float>(ph));
-                    _Float16* pr = pq + (static_cast<size_t>(row) * (k / 256) + blk / 8) * 16 + (blk & 7);
-                    pr[0] = ph;
-                    pr[8] = pl;
-                }
-            }
-        }
-    };
+    auto emit = [&](const float4 v, int32_t t) { emit_q(v, t, row, k, inv, xq, dxs, pq); };
     // whole 8-lane groups take the same branches and trip counts (tasks and
     // NT are multiples of 8), as the group operations need
 #pragma unroll
-    for (int u = 0; u < kHiloU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int32_t t = static_cast<int32_t>(threadIdx.x) + u * NT;
         if (t < tasks) emit(xv[u], t);
     }
-    for (int32_t t = threadIdx.x + kHiloU * NT; t < tasks; t += NT) emit(xr[t], t);
+    for (int32_t t = threadIdx.x + U * NT; t < tasks; t += NT) emit(xr[t], t);
 }
 
-// the streamed kernel's activations: q as fp16 [B x K], then the blocks'
-// d / s [B x K / 32] (dxs), the P pairs (Q4_K) and the row scales
-void launch_act_q(const float* x, int32_t b, int32_t k, _Float16* xq, float* dxs, float* rscale, _Float16* pq,
-                  hipStream_t stream, const float* up) {
-    uint2* o = reinterpret_cast<uint2*>(xq);
+// A call's buffers in the workspace: q [B x K] and the blocks' d / s [B x K /
+// 32], P (Q4_K, else null), the row scales, the split-K partials
+struct QsBufs {
+    _Float16* xq;
+    float* dxs;
+    _Float16* pq;
+    float* rscale;
+    float* part;
+};
+
+// up non-null: the rows are SwiGLU(x, up)
+void launch_act_q(const float* x, int32_t b, int32_t k, const QsBufs& q, hipStream_t stream, const float* up) {
+    uint2* o = reinterpret_cast<uint2*>(q.xq);
     if (up) {
         if (k <= 4 * 4 * kThreads)
-            hipLaunchKernelGGL((act_hilo_kernel<4, true, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale,
-                               pq, up, dxs);
+            hipLaunchKernelGGL((act_q_kernel<4, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, q.rscale, q.pq,
+                               up, q.dxs);
         else if (k <= 3 * 4 * 1024)  // up to 12288-wide rows: 16 waves, 3 float4 pairs each
-            hipLaunchKernelGGL((act_hilo_kernel<3, true, true, 1024>), dim3(b), dim3(1024), 0, stream, x, k, o,
-                               rscale, pq, up, dxs);
+            hipLaunchKernelGGL((act_q_kernel<3, true, 1024>), dim3(b), dim3(1024), 0, stream, x, k, o, q.rscale,
+                               q.pq, up, q.dxs);
         else
-            hipLaunchKernelGGL((act_hilo_kernel<16, true, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale,
-                               pq, up, dxs);
+            hipLaunchKernelGGL((act_q_kernel<16, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, q.rscale, q.pq,
+                               up, q.dxs);
+    } else if (b <= 512 && k > 2048 && k <= 4 * 4 * 1024) {
+        // few long rows: 16 waves each (4096 x 1438 at K = 5504, B = 113: 36.2 ->
+        // 30.4 us with the paired stores below; rows up to 2048 gain nothing)
+        if (k <= 4 * 1024)
+            hipLaunchKernelGGL((act_q_kernel<1, false, 1024>), dim3(b), dim3(1024), 0, stream, x, k, o, q.rscale, q.pq,
+                               nullptr, q.dxs);
+        else
+            hipLaunchKernelGGL((act_q_kernel<4, false, 1024>), dim3(b), dim3(1024), 0, stream, x, k, o, q.rscale, q.pq,
+                               nullptr, q.dxs);
     } else if (k <= 4 * 4 * kThreads) {
-        hipLaunchKernelGGL((act_hilo_kernel<4, false, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale, pq,
-                           nullptr, dxs);
+        hipLaunchKernelGGL((act_q_kernel<4>), dim3(b), dim3(kThreads), 0, stream, x, k, o, q.rscale, q.pq, nullptr,
+                           q.dxs);
     } else {
-        hipLaunchKernelGGL((act_hilo_kernel<16, false, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale,
-                           pq, nullptr, dxs);
+        hipLaunchKernelGGL((act_q_kernel<16>), dim3(b), dim3(kThreads), 0, stream, x, k, o, q.rscale, q.pq, nullptr,
+                           q.dxs);
     }
 }
 
@@ -256,7 +215,7 @@ void launch_act_q(const float* x, int32_t b, int32_t k, _Float16* xq, float* dxs
 // (elementwise.hip) with its thread layout (1024 threads, float4 t = thread +
 // 1024 j, up to 4 per thread), sum order and operation order, so the rows
 // quantised are those gncx_hip_add_rmsnorm_rows / gncx_hip_rmsnorm_rows
-// write; the quantisation is act_hilo_kernel's (a row maximum, then 8
+// write; the quantisation is act_q_kernel's (a row maximum, then 8
 // consecutive lanes per 32-block).
 constexpr int kNaThreads = 1024;
 constexpr int kNaRegs = 4;
@@ -322,7 +281,7 @@ __global__ __launch_bounds__(kNaThreads) void norm_act_q_kernel(const float* x, 
 #pragma unroll
     for (int j = 0; j < kNaRegs; ++j) {
         const int32_t t = tid + kNaThreads * j;
-        if (t < n4) emit_qx(yv[j], t, row, k, inv, xq, dxs, pq);
+        if (t < n4) emit_q(yv[j], t, row, k, inv, xq, dxs, pq);
     }
 }
 
@@ -333,470 +292,20 @@ bool norm_act_fits(const float* h, const float* r, const float* gamma, int32_t k
     return k > 0 && k % 256 == 0 && k / 4 <= kNaThreads * kNaRegs && (al & 15u) == 0;
 }
 
-void launch_norm_act_q(float* h, const float* r, const float* gamma, float eps, int32_t b, int32_t k, _Float16* xq,
-                       float* dxs, float* rscale, _Float16* pq, hipStream_t stream) {
-    uint2* o = reinterpret_cast<uint2*>(xq);
+void launch_norm_act_q(float* h, const float* r, const float* gamma, float eps, int32_t b, int32_t k,
+                       const QsBufs& q, hipStream_t stream) {
+    uint2* o = reinterpret_cast<uint2*>(q.xq);
     if (r)
         hipLaunchKernelGGL(norm_act_q_kernel<true>, dim3(b), dim3(kNaThreads), 0, stream, h, r, h, gamma, k, eps, o,
-                           dxs, rscale, pq);
+                           q.dxs, q.rscale, q.pq);
     else
         hipLaunchKernelGGL(norm_act_q_kernel<false>, dim3(b), dim3(kNaThreads), 0, stream, h, nullptr, nullptr,
-                           gamma, k, eps, o, dxs, rscale, pq);
+                           gamma, k, eps, o, q.dxs, q.rscale, q.pq);
 }
 
-// up non-null: the rows are SwiGLU(x, up)
-void launch_act_hilo(const float* x, int32_t b, int32_t k, _Float16* xhl, float* rscale, _Float16* pq,
-                     hipStream_t stream, const float* up = nullptr) {
-    uint2* o = reinterpret_cast<uint2*>(xhl);
-    if (up) {
-        if (k <= 4 * 4 * kThreads)
-            hipLaunchKernelGGL((act_hilo_kernel<4, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale, pq, up);
-        else
-            hipLaunchKernelGGL((act_hilo_kernel<16, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale, pq,
-                               up);
-    } else if (k <= 4 * 4 * kThreads) {
-        hipLaunchKernelGGL((act_hilo_kernel<4>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale, pq, nullptr);
-    } else {
-        hipLaunchKernelGGL((act_hilo_kernel<16>), dim3(b), dim3(kThreads), 0, stream, x, k, o, rscale, pq, nullptr);
-    }
-}
-
-// Weights e0 .. e0 + 15 (e0 a multiple of 16) of one row: raw block bytes
-// loaded into registers (WSeg::load, issued two K steps ahead of their use),
-// then dequantised in fp32 (WSeg::get) and split into fp16 pairs on their way
-// into LDS; an all-zero block (what a past-the-end buffer load reads)
-// dequantises to zeros.  Formulas: Q4_0 d (q - 8), elements j and j + 16 in
-// the low and high nibbles of byte j (cpp:1023-1030); Q8_0 d q; Q4_K
-// (d sc) q - dmin m with sub-block j of chunk c in the low (j even) or high
-// nibbles of bytes 32c .. 32c + 31 (cpp:1135-1178); Q6_K (d sc) (q - 32) with
-// element l + 32 g of a 128-half from ql[l + 32 (g & 1)] (nibble g / 2),
-// qh[l] >> 2g and scale l / 16 + 2g (cpp:742-757).
-template <int TYPE>
-struct WSeg;
-
-template <>
-struct WSeg<kQ4_0> {
-    uint32_t d, sh;
-    Raw16 qs;
-    template <class Row>
-    __device__ __forceinline__ void load(const Row& r, int32_t e0) {
-        const uint32_t blk = static_cast<uint32_t>(e0 / 32) * 18u;
-        d = r.ldu16(blk);
-        sh = r.sh(blk + 2u);
-        raw16_load(qs, r, blk + 2u, sh);
-    }
-    __device__ __forceinline__ void get(int32_t e0, float (&v)[16]) const {
-        const float dv = half_bits_to_float(d);
-        const uint4 q = raw16_get(qs, sh);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        const int s = 4 * ((e0 >> 4) & 1);
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            v[i] = dv * static_cast<float>(static_cast<int>((w[i >> 2] >> (s + 8 * (i & 3))) & 15u) - 8);
-    }
-};
-
-template <>
-struct WSeg<kQ8_0> {
-    uint32_t d, sh;
-    Raw16 qs;
-    template <class Row>
-    __device__ __forceinline__ void load(const Row& r, int32_t e0) {
-        const uint32_t blk = static_cast<uint32_t>(e0 / 32) * 34u;
-        d = r.ldu16(blk);
-        const uint32_t o = blk + 2u + 16u * static_cast<uint32_t>((e0 >> 4) & 1);
-        sh = r.sh(o);
-        raw16_load(qs, r, o, sh);
-    }
-    __device__ __forceinline__ void get(int32_t, float (&v)[16]) const {
-        const float dv = half_bits_to_float(d);
-        const uint4 q = raw16_get(qs, sh);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            v[i] = dv * static_cast<float>(static_cast<int8_t>((w[i >> 2] >> (8 * (i & 3))) & 0xffu));
-    }
-};
-
-template <>
-struct WSeg<kQ4_K> {
-    u32x4 hdr, q;
-    template <class Row>
-    __device__ __forceinline__ void load(const Row& r, int32_t e0) {
-        const uint32_t blk = static_cast<uint32_t>(e0 / 256) * 144u, rr = static_cast<uint32_t>(e0 % 256);
-        hdr = r.ld16(blk);
-        q = r.ld16(blk + 16u + 32u * (rr / 64u) + (rr % 32u));
-    }
-    __device__ __forceinline__ void get(int32_t e0, float (&v)[16]) const {
-        const int j = (e0 % 256) / 32, s = 4 * (j & 1);
-        int sc, mn;
-        k4_scale_min(j, hdr.y, hdr.z, hdr.w, sc, mn);
-        const float a = half_bits_to_float(hdr.x & 0xffffu) * static_cast<float>(sc);
-        const float m = half_bits_to_float(hdr.x >> 16) * static_cast<float>(mn);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = a * static_cast<float>((w[i >> 2] >> (s + 8 * (i & 3))) & 15u) - m;
-    }
-};
-
-template <>
-struct WSeg<kQ6_K> {
-    Raw16 ql, qh;
-    uint32_t scw, d, sh;
-    template <class Row>
-    __device__ __forceinline__ void load(const Row& r, int32_t e0) {
-        const uint32_t blk = static_cast<uint32_t>(e0 / 256) * 210u;
-        const uint32_t rr = static_cast<uint32_t>(e0 % 256), h = rr / 128u, g = (rr % 128u) / 32u, l0 = rr % 32u;
-        sh = r.sh(blk);  // every field offset used here is even: one shift for all
-        raw16_load(ql, r, blk + 64u * h + 32u * (g & 1u) + l0, sh);
-        raw16_load(qh, r, blk + 128u + 32u * h + l0, sh);
-        scw = r.ldu16(blk + 192u + 8u * h + 2u * g);  // scales l0 / 16 + 2g of this half
-        d = r.ldu16(blk + 208u);
-    }
-    // sc (q - 32) as integers, |sc (q - 32)| <= 4096 (d is applied per
-    // super-block); returns sc
-    __device__ __forceinline__ int get_int(int32_t e0, int (&v)[16]) const {
-        const int rr = e0 % 256, g = (rr % 128) / 32, l0 = rr % 32;
-        const int sc = static_cast<int8_t>((scw >> (l0 >= 16 ? 8 : 0)) & 0xffu);
-        const uint4 a = raw16_get(ql, sh), b = raw16_get(qh, sh);
-        const uint32_t L[4] = {a.x, a.y, a.z, a.w}, H[4] = {b.x, b.y, b.z, b.w};
-        const int lsh = 4 * (g >> 1), hsh = 2 * g;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int sh8 = 8 * (i & 3);
-            const int q = static_cast<int>(((L[i >> 2] >> (lsh + sh8)) & 15u) | (((H[i >> 2] >> (hsh + sh8)) & 3u) << 4));
-            v[i] = sc * (q - 32);
-        }
-        return sc;
-    }
-    __device__ __forceinline__ void get(int32_t e0, float (&v)[16]) const {
-        const int rr = e0 % 256, g = (rr % 128) / 32, l0 = rr % 32;
-        const float s = half_bits_to_float(d) * static_cast<float>(static_cast<int8_t>((scw >> (l0 >= 16 ? 8 : 0)) & 0xffu));
-        const uint4 a = raw16_get(ql, sh), b = raw16_get(qh, sh);
-        const uint32_t L[4] = {a.x, a.y, a.z, a.w}, H[4] = {b.x, b.y, b.z, b.w};
-        const int lsh = 4 * (g >> 1), hsh = 2 * g;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int sh8 = 8 * (i & 3);
-            const int q = static_cast<int>(((L[i >> 2] >> (lsh + sh8)) & 15u) | (((H[i >> 2] >> (hsh + sh8)) & 3u) << 4));
-            v[i] = s * static_cast<float>(q - 32);
-        }
-    }
-};
-
-// Y tile of (32 WM MW) tokens x (64 WN) rows per work-group of 2 MW waves
-// (MW along the tokens, 2 along the rows); each wave owns WM x WN 32x32
-// accumulator tiles.  Both operands are fp16 pairs (hi, lo), and each 16-wide
-// K slice runs three v_mfma_f32_32x32x16_f16 per tile: x_hi w_hi + x_lo w_hi +
-// x_hi w_lo (x_lo w_lo is below 2^-22 of the product).  With fp32
-// accumulation the result is within about 2e-7 relative L2 of the
-// reference's integer block dots (measured on the CPU and the GPU for all
-// four formats), where fp16 operands alone reach 3e-4.
-// K advances 32 per step through two LDS buffers, each holding token rows
-// [tokens][32 + 8 pad] and weight rows [rows][32 + 8 pad] as hi and lo
-// arrays.  In step s the MFMAs consume buffer s % 2 while the loads for
-// later steps are in flight, then step s + 1's registers are written to the
-// other buffer; one barrier per step.  All loads are buffer loads whose
-// out-of-range reads return 0 without a memory request (tokens past B, K past
-// the range, rows past N), so each wave issues the same loads every step and
-// each wait covers exactly the loads it needs.
-// MFMA operand layouts (v_mfma_f32_32x32x16_f16): lane l holds
-// A[l % 32][8 (l / 32) .. + 8] and B[8 (l / 32) .. + 8][l % 32]; accumulator
-// register r of lane l is D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
-// blockIdx.z selects a K range of kchunk (split K); with gridDim.z > 1 the
-// tile goes to part[z][t][m] and matbatch_reduce_kernel adds the ranges in
-// order.
-// Q6_K weights are d (sc (q - 32)) (cpp:742-757) with sc (q - 32) an integer
-// of magnitude at most 4096 and d fixed over a 256-value super-block, so the
-// weight operand is that integer: exact in fp16 up to 2048 (|sc| <= 64),
-// else its fp16 rounding (hi) plus an exact remainder of -1, 0 or 1 (lo).
-// On the 256-token tiles (B > 128) the products of a super-block go to a
-// second accumulator D, folded in as
-// acc += d D at its end (d of the lane's weight row), and x_hi w_lo, the
-// third product, runs only in steps where some weight of the tile has
-// |sc| > 64: elsewhere w_lo is zero.  The third product's step flag is the
-// step's first K index, written to LDS by any thread that dequantised such
-// a scale (a stale flag never equals a later step's index).
-constexpr int kMfKs = 32;
-constexpr int kMfLd = kMfKs + 8;  // halves per LDS row (16-byte aligned, staggers banks)
 // a buffer offset past any resource (resources here are below 2^30 bytes);
 // small field offsets may still be added to it without leaving int32
 constexpr int32_t kMfOob = 0x7ff00000;
-
-template <int WM, int WN, int MW>
-constexpr size_t mfma_lds_bytes() {
-    return 2 * 2 * static_cast<size_t>(32 * WM * MW + 64 * WN) * kMfLd * sizeof(_Float16);
-}
-
-template <int TYPE, int WM, int WN, int MW = 2>
-__global__ __launch_bounds__(128 * MW, MW == 2 ? 2 : 1) void matbatch_mfma_kernel(const uint8_t* __restrict w,
-                                                                                   size_t rbytes,
-                                                            const _Float16* __restrict xhl,
-                                                            const float* __restrict rscale, int32_t b, int32_t k,
-                                                            int32_t n, float* __restrict y, int32_t kchunk,
-                                                            float* __restrict part) {
-    constexpr int THREADS = 128 * MW;
-    constexpr int BM = 32 * WM * MW, BN = 64 * WN;
-    static_assert(2 * BN <= THREADS, "one thread per 16-value weight piece of a step");
-    constexpr int XCH = BM * 4 / THREADS;  // 16-byte chunks of 8 values (hi and lo each) per thread and step
-    static_assert(XCH * THREADS == BM * 4, "whole chunks per thread");
-    static_assert(mfma_lds_bytes<WM, WN, MW>() <= 160 * 1024, "LDS of one CU");
-    __shared__ __align__(16) _Float16 xs[2][2][BM * kMfLd];  // [buffer][hi, lo]
-    __shared__ __align__(16) _Float16 ws[2][2][BN * kMfLd];
-    // The tile's token scales sit in the padding of the activation rows of
-    // buffer 1 (halves kMfKs .. kMfLd of row r, which no load, store or
-    // product touches), so they cost no LDS: 64x64 tiles fill the CU's LDS
-    // with four work-groups at exactly 40 KB each.  Read from memory at the
-    // output, they were a dependent load of every wave at the moment all
-    // work-groups store.
-    static_assert(kMfLd - kMfKs >= 2 && BM <= THREADS, "a float of padding per row, one scale per thread");
-    auto rs_at = [&](int r) -> float& { return *reinterpret_cast<float*>(&xs[1][0][r * kMfLd + kMfKs]); };
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = wv % MW, wn = wv / MW;
-    const int32_t t0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int32_t kb = blockIdx.z * kchunk;
-    const int32_t ke = min(k, kb + kchunk);
-    const int32_t nsteps = (ke - kb + kMfKs - 1) / kMfKs;
-
-    // (the 256-token tiles only: on the smaller ones D's registers cost
-    // occupancy, measured 5-11% slower at B = 16 to 100)
-    constexpr bool Q6 = TYPE == kQ6_K && MW == 4;
-    // Q6_K: d of the tile's rows per super-block parity, the third-product flags
-    __shared__ float q6d[Q6 ? 2 : 1][Q6 ? BN : 1];
-    __shared__ int32_t q6big[2];
-    floatx16 acc[WM][WN], D[Q6 ? WM : 1][Q6 ? WN : 1];
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    if constexpr (Q6) {
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) D[i][j][r] = 0.0f;
-    }
-
-    // activation chunks c = tid + THREADS i: token row c / 4 of the tile,
-    // values 8 (c % 4) .. + 8 of the step, hi at byte 32 j and lo at 32 j + 16
-    // of chunk j = (row k + value) / 8; one resource over the tile's token rows
-    const int32_t rows_here = min(BM, b - t0);
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16*>(xhl + static_cast<size_t>(t0) * k * 2), static_cast<short>(0),
-        rows_here * k * 2 * static_cast<int32_t>(sizeof(_Float16)), 0x00020000);
-    // weight piece tid (row tid / 2 of the tile, 16 values at 16 (tid % 2))
-    // for tid < 2 BN, through one resource over the tile's rows
-    const int wrow = tid >> 1, wseg = tid & 1;
-    const int32_t wrows_here = min(BN, n - n0);
-    TileRow wrs;
-    wrs.r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + static_cast<size_t>(n0) * rbytes),
-                                              static_cast<short>(0),
-                                              wrows_here * static_cast<int32_t>(rbytes), 0x00020000);
-    wrs.base = tid < 2 * BN && wrow < wrows_here ? wrow * static_cast<int32_t>(rbytes) : kMfOob / 2;
-
-    uint4 xr[XCH][2];
-    WSeg<TYPE> wr[2];
-    // activation chunks of one step; past the range an offset past the
-    // resource reads zeros
-    auto gload_x = [&](int32_t k0) {
-#pragma unroll
-        for (int i = 0; i < XCH; ++i) {
-            const int c = tid + THREADS * i, r = c >> 2, seg = c & 3;
-            const int32_t kx = k0 + 8 * seg;
-            const int32_t off = kx < ke ? (r * k + kx) * 2 * static_cast<int32_t>(sizeof(_Float16)) : kMfOob;
-            const u32x4 h = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
-            const u32x4 l = __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16, 0, 0);
-            xr[i][0] = make_uint4(h.x, h.y, h.z, h.w);
-            xr[i][1] = make_uint4(l.x, l.y, l.z, l.w);
-        }
-    };
-    // raw weight blocks of one step into register set `set`; past the range
-    // (k, ke are multiples of 32) the row base moves past the resource, so
-    // every field reads zeros without a memory request
-    auto gload_w = [&](int set, int32_t k0) {
-        const int32_t kw = k0 + 16 * wseg;
-        TileRow r = wrs;
-        if (kw >= ke) r.base = kMfOob / 2;
-        wr[set].load(r, kw < ke ? kw : 0);
-    };
-    auto lstore = [&](int set, int buf, int32_t k0) {
-#pragma unroll
-        for (int i = 0; i < XCH; ++i) {
-            const int c = tid + THREADS * i, r = c >> 2, seg = c & 3;
-            *reinterpret_cast<uint4*>(&xs[buf][0][r * kMfLd + 8 * seg]) = xr[i][0];
-            *reinterpret_cast<uint4*>(&xs[buf][1][r * kMfLd + 8 * seg]) = xr[i][1];
-        }
-        if (tid < 2 * BN) {
-            const int32_t kw = k0 + 16 * wseg;
-            uint32_t hi[8], lo[8];
-            if constexpr (Q6) {
-                int v[16];
-                const int sc = wr[set].get_int(kw < ke ? kw : 0, v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const _Float16 h0 = static_cast<_Float16>(static_cast<float>(v[2 * i]));
-                    const _Float16 h1 = static_cast<_Float16>(static_cast<float>(v[2 * i + 1]));
-                    const _Float16 l0 = static_cast<_Float16>(static_cast<float>(v[2 * i]) - static_cast<float>(h0));
-                    const _Float16 l1 =
-                        static_cast<_Float16>(static_cast<float>(v[2 * i + 1]) - static_cast<float>(h1));
-                    hi[i] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h0)) |
-                            (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h1)) << 16);
-                    lo[i] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l0)) |
-                            (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l1)) << 16);
-                }
-                if (sc > 64 || sc < -64) q6big[buf] = k0;
-                // a super-block's first step in this range stores the rows' d
-                if (wseg == 0 && (k0 == kb || k0 % 256 == 0))
-                    q6d[(k0 / 256) & 1][wrow] = half_bits_to_float(kw < ke ? wr[set].d : 0u);
-            } else {
-                float v[16];
-                wr[set].get(kw < ke ? kw : 0, v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) split2(v[2 * i], v[2 * i + 1], hi[i], lo[i]);
-            }
-            uint4* dh = reinterpret_cast<uint4*>(&ws[buf][0][wrow * kMfLd + 16 * wseg]);
-            uint4* dl = reinterpret_cast<uint4*>(&ws[buf][1][wrow * kMfLd + 16 * wseg]);
-            dh[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-            dh[1] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-            dl[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            dl[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
-        }
-    };
-
-    const int li = lane & 31, lk = 8 * (lane >> 5);
-    // Q6_K: products into D, the third only where a weight has |sc| > 64;
-    // D folded into acc with d at a super-block's last step in the range
-    auto compute_q6 = [&](int buf, int32_t k0) {
-        const bool third = q6big[buf] == k0;
-#pragma unroll
-        for (int kk = 0; kk < kMfKs; kk += 16) {
-            half8 ah[WM], al[WM], bh[WN];
-#pragma unroll
-            for (int i = 0; i < WM; ++i) {
-                const int o = (wm * 32 * WM + 32 * i + li) * kMfLd + kk + lk;
-                ah[i] = *reinterpret_cast<const half8*>(&xs[buf][0][o]);
-                al[i] = *reinterpret_cast<const half8*>(&xs[buf][1][o]);
-            }
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-                bh[j] = *reinterpret_cast<const half8*>(&ws[buf][0][(wn * 32 * WN + 32 * j + li) * kMfLd + kk + lk]);
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], D[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], D[i][j], 0, 0, 0);
-            if (third) {
-                half8 bl[WN];
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    bl[j] =
-                        *reinterpret_cast<const half8*>(&ws[buf][1][(wn * 32 * WN + 32 * j + li) * kMfLd + kk + lk]);
-#pragma unroll
-                for (int i = 0; i < WM; ++i)
-#pragma unroll
-                    for (int j = 0; j < WN; ++j)
-                        D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], D[i][j], 0, 0, 0);
-            }
-        }
-        if ((k0 + kMfKs) % 256 == 0 || k0 + kMfKs >= ke) {
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const float dv = q6d[(k0 / 256) & 1][wn * 32 * WN + 32 * j + li];
-#pragma unroll
-                for (int i = 0; i < WM; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        acc[i][j][r] = fmaf(D[i][j][r], dv, acc[i][j][r]);
-                        D[i][j][r] = 0.0f;
-                    }
-            }
-        }
-    };
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int kk = 0; kk < kMfKs; kk += 16) {
-            half8 ah[WM], al[WM], bh[WN], bl[WN];
-#pragma unroll
-            for (int i = 0; i < WM; ++i) {
-                const int o = (wm * 32 * WM + 32 * i + li) * kMfLd + kk + lk;
-                ah[i] = *reinterpret_cast<const half8*>(&xs[buf][0][o]);
-                al[i] = *reinterpret_cast<const half8*>(&xs[buf][1][o]);
-            }
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const int o = (wn * 32 * WN + 32 * j + li) * kMfLd + kk + lk;
-                bh[j] = *reinterpret_cast<const half8*>(&ws[buf][0][o]);
-                bl[j] = *reinterpret_cast<const half8*>(&ws[buf][1][o]);
-            }
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-        }
-    };
-
-    // Activations are loaded one step ahead, raw weight blocks two steps
-    // ahead in two register sets.  Each step issues the activation loads
-    // before the weight loads: loads retire in order, so the wait before
-    // writing step s + 1 to LDS does not cover step s + 2's weights.  Steps go
-    // in pairs so that register-set and buffer indices are compile-time
-    // constants; loads past the range read nothing.
-    // the scale load goes first: the wait for step 0's loads covers it
-    const float rsv = tid < rows_here ? rscale[t0 + tid] : 1.0f;
-    gload_x(kb);
-    gload_w(0, kb);
-    gload_w(1, kb + kMfKs);
-    lstore(0, 0, kb);
-    if (tid < BM) rs_at(tid) = rsv;
-    __syncthreads();
-    for (int32_t s = 0; s < nsteps; s += 2) {
-        const int32_t k0 = kb + s * kMfKs;
-        gload_x(k0 + kMfKs);
-        gload_w(0, k0 + 2 * kMfKs);
-        if constexpr (Q6) compute_q6(0, k0);
-        else compute(0);
-        if (s + 1 < nsteps) lstore(1, 1, k0 + kMfKs);
-        __syncthreads();
-        if (s + 1 >= nsteps) break;
-        gload_x(k0 + 2 * kMfKs);
-        gload_w(1, k0 + 3 * kMfKs);
-        if constexpr (Q6) compute_q6(1, k0 + kMfKs);
-        else compute(1);
-        if (s + 2 < nsteps) lstore(0, 0, k0 + 2 * kMfKs);
-        __syncthreads();
-    }
-    float* dst = gridDim.z > 1 ? part + static_cast<size_t>(blockIdx.z) * b * n : y;
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            const int32_t mm = n0 + wn * 32 * WN + 32 * j + li;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int32_t t = t0 + wm * 32 * WM + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (t < b && mm < n) dst[static_cast<size_t>(t) * n + mm] = acc[i][j][r] * rs_at(t - t0);
-            }
-        }
-}
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
@@ -842,94 +351,252 @@ struct RedMats {
     int32_t count;
 };
 
-// ---- Q4_K and Q6_K, weights streamed through registers ------------------------
+// ---- quantised weights, streamed through registers ------------------------------
 //
-// A work-group is RT row tiles of 32 weight rows (one wave each) times 64
-// tokens.  Each wave streams its rows' super-blocks straight from memory
-// into registers, a super-block ahead: lane l holds row l % 32 and bytes
-// 16 h .. 16 h + 15 (h = l / 32) of each sub-block pair's 32 qs bytes, i.e.
-// values 16 h .. 16 h + 15 of both sub-blocks, which dequantised to sc q
-// are its A operands of v_mfma_f32_32x32x16_f16: K slice s of a sub-block
-// is values 16 h + 8 s .. + 8 in lane half h, and the activation operand is
-// read from LDS in the same order, so each slice's products pair every
-// value with its own activation.  The activations (q as fp16, the blocks'
-// d / s and, for the min term, the P pairs) stream through three LDS
-// stages, one super-block per stage, filled by direct-to-LDS loads two
-// super-blocks ahead, issued with the next super-block's weights as a
-// super-block starts; one barrier per super-block.  Each block's
-// integer dot is one product, scaled on the VALU by the block's d_x / s into
-// a super-block accumulator, and d, dmin and the min term fold once per
-// super-block.  No weight is staged in LDS and nothing is barriered per 32
-// values: a work-group's weights are read once, by the wave that uses them.
-// With gridDim.z > 1 the work-group's result is a split-K partial.
-// The result leaves through LDS, so that each store instruction writes one
-// token's contiguous row range.
-// Q6_K (cpp:742-757) takes the same structure: the weights are the integers
-// sc (q - 32), d folds once per super-block and there is no min term.
-// sc (q - 32) can need 12 bits (|sc| up to 128), so each is taken as two
-// fp16 integers that are always exact, sc (l - 16) and 16 sc (u - 1) (q = l
-// + 16 u, l the 4 bits from ql, u the 2 from qh), and a block's dot is two
-// products per K slice (integers below 2^24: exact).  Lane half h takes
-// values 16 h .. 16 h + 15 of each 32-value group of both 128-value halves:
-// per half the 16 bytes of ql at 16 h and at 32 + 16 h and of qh at 16 h
-// (all four groups' values), so a group's two K slices are again values
-// 16 h + 8 s .. + 8.  Its blocks are only 2-byte aligned: each 16-byte piece
-// is read as a dwordx4 from the dword at or below it plus one dword, and
-// realigned.
-constexpr int kQsTok = 64;            // tokens per work-group
-constexpr int kQsXHalves = 64 * 260;  // halves per q stage: 64 x 256 of q, or 32 x (256 + 4) floats of output
+// A work-group is 8 waves of 32 weight rows (two 16-row fragments) times 16
+// TF tokens.  Each wave streams its rows' super-blocks (256 values; eight
+// blocks of Q8_0 / Q4_0) straight from memory into registers, a super-block
+// ahead; nothing about the weights goes through LDS but the rows' scales.
+// One v_mfma_f32_16x16x32_f16 is one 32-value block of a 16 x 16 tile: lane
+// l holds row (A operand, weights) or token (B, activations) l % 16 and
+// values 8 g .. 8 g + 7 of the block, g = l / 16, in the order 0 2 1 3 4 6 5
+// 7 on both sides (the order in which masks pick byte pairs out of a dword).
+// Weights are small integers, exact in fp16, and activations the quantised q,
+// so a block's product is its exact integer dot (below 2^24).  The block
+// scales are applied on the VALU: S += (d_x / s) dot, where d of Q8_0 / Q4_0
+// (one per row and block) goes in with d_x, and per super-block acc += d S
+// (Q4_K: - dmin (m . P)).  Weights:
+//   Q4_K  sc q, from the fp16 integers 1024 + q (or 1024 + 16 q for the high
+//         nibbles, with sc / 16): one mask-or and one packed fma per pair
+//   Q6_K  sc (q - 32) can need 12 bits (|sc| up to 128), so two products: sc
+//         (l - 16) and 16 sc (u - 1) (q = l + 16 u: the 4 bits from ql, the 2
+//         from qh), integers exact in fp16 for every int8 scale, from the fp16
+//         values 16 + l and 4 + u with one fma each
+//   Q8_0  q, Q4_0  q - 8
+// Tiles of 16 x 16 rather than 32 x 32: a block is one instruction instead of
+// two dependent ones, and its 4 result registers per tile leave room to scale
+// one tile while the next ones multiply, and so for 128 tokens per wave, which
+// halves the weights' unpacking and loads per output.
+// Full calls at 4096 x 12288, B = 2048 / 512, before (32 x 32 tiles of 64
+// tokens; Q8_0 and Q4_0: both operands as fp16 pairs, three products) and
+// now: Q4_K 413 / 130 -> 310 / 105 us, Q6_K 665 / 213 -> 452 / 146, Q8_0 650 /
+// 200 -> 425 / 140, Q4_0 635 / 196 -> 417 / 136; 64-token tiles 382 / 128 (Q4_K).
+// Bound (counters, Q4_K at B = 2048): VALU issue 62% of the cycles (512 of 846
+// instructions per wave and super-block are the block scales), LDS 50%, matrix
+// cores 32%, at a clock of 2.08 GHz.  With work taken out in a copy, 335 us
+// became 245 without the activation reads from LDS, 209 without products,
+// 280 without the scales, 311 without the unpacking.
+//
+// The activations (q as fp16, d_x / s per block and, for the min term, P
+// pairs) stream through three LDS stages, one super-block each, filled by
+// direct-to-LDS loads two super-blocks ahead; one barrier per super-block.
+// With gridDim.z > 1 the result is a split-K partial.  It leaves through LDS,
+// so that each store instruction writes one token's contiguous row range.
+constexpr int kQsRows = 256;  // weight rows per work-group
 
-// one super-block of a lane's weight row in registers
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ half2 h2_of(uint32_t v) { return __builtin_bit_cast(half2, v); }
+__device__ __forceinline__ uint32_t u_of(half2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ half2 h2_all(float v) { return half2{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
+
+// One super-block of a lane's weight row in registers: the bytes that hold
+// its 8 values of each block, and the scales.  A register is loaded again,
+// for the next super-block, as soon as its last block's operands are formed:
+// load<P>(byte offset, lane group g, further blocks of the row) issues the
+// loads of part P, -1 for the scales and j for what block j uses last.
+// Blocks past the row (Q8_0, Q4_0: nblk) read zeros.
 template <int TYPE>
 struct QsW;
 template <>
 struct QsW<kQ4_K> {
     static constexpr int32_t kBytes = 144;
-    u32x4 h, q[4];  // header; 16 bytes of each sub-block pair's qs
-    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int lh) {
-        h = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) q[p] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 + 32 * p + 16 * lh, 0, 0);
+    static constexpr int kLoads = 5;
+    u32x4 h;
+    u32x2 q[4];  // bytes 8 g .. of each sub-block pair's 32
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t) {
+        if constexpr (P == -1) h = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+        else if constexpr ((P & 1) == 1)
+            q[P >> 1] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 16 + 16 * (P - 1), 0, 0);
     }
 };
 template <>
 struct QsW<kQ6_K> {
     static constexpr int32_t kBytes = 210;
-    // pieces: ql of half 0 at 16 h and 32 + 16 h, of half 1 at 64 + 16 h and
-    // 96 + 16 h, qh at 128 + 16 h and 160 + 16 h, the scales and d at 192;
-    // each as the 20 bytes from the dword at or below it
-    u32x4 p[7];
-    uint32_t e[7];
-    static __device__ __forceinline__ int32_t piece(int i, int lh) {
-        return i < 6 ? 32 * i + 16 * lh : 192;
+    static constexpr int kLoads = 8;
+    u32x4 s;           // the 16 scales
+    u32x2 l[4], u[2];  // ql bytes 8 g .. of each 32, qh bytes 8 g .. of each 32
+    uint32_t d;
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t) {
+        if constexpr (P == -1) {
+            s = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 192, 0, 0);
+            d = __builtin_amdgcn_raw_buffer_load_b16(rs, off + 208, 0, 0);
+        } else if constexpr ((P & 2) == 2) {
+            constexpr int i = 2 * (P >> 2) + (P & 1);
+            l[i] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 32 * i, 0, 0);
+            if constexpr ((P & 1) == 1)
+                u[P >> 2] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 128 + 32 * (P >> 2), 0, 0);
+        }
     }
-    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int lh) {
+};
+template <>
+struct QsW<kQ8_0> {
+    static constexpr int32_t kBytes = 272;
+    static constexpr int kLoads = 10;
+    u32x2 q[8];
+    uint32_t d[2];  // of blocks 2 g and 2 g + 1
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
+        if constexpr (P == -1) {
 #pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            const int32_t o = (off + piece(i, lh)) & ~3;
-            p[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0);
-            e[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, o + 16, 0, 0);
+            for (int e = 0; e < 2; ++e)
+                d[e] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * g + e < nblk ? off + 34 * (2 * g + e) : kMfOob, 0, 0);
+        } else {
+            q[P] = __builtin_amdgcn_raw_buffer_load_b64(rs, P < nblk ? off + 8 * g + 34 * P + 2 : kMfOob, 0, 0);
+        }
+    }
+};
+template <>
+struct QsW<kQ4_0> {
+    static constexpr int32_t kBytes = 144;
+    static constexpr int kLoads = 10;
+    u32x2 q[8];  // bytes 8 (g % 2) .. of each block's 16
+    uint32_t d[2];
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
+        if constexpr (P == -1) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                d[e] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * g + e < nblk ? off + 18 * (2 * g + e) : kMfOob, 0, 0);
+        } else {
+            q[P] = __builtin_amdgcn_raw_buffer_load_b64(rs, P < nblk ? off + 8 * (g & 1) + 18 * P + 2 : kMfOob, 0, 0);
         }
     }
 };
 
-template <int TYPE, int RT>
-__global__ __launch_bounds__(64 * RT, 1) void matbatch_qs_stream_kernel(
+// (v & mask) | e as one v_and_or_b32: with e hidden in a vector register and
+// the mask in a scalar one (two literals would take two instructions)
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// The A operands of a lane's row for one super-block: prepare() unpacks what
+// all blocks share, get(w, g, j, d, o) forms dword d (0, 1) of block j's
+// operand, 4 of its 8 values (o.b: Q6_K's second product).
+struct QsOut {
+    uint32_t a[4], b[4];
+};
+template <int TYPE>
+struct QsOperand;
+template <>
+struct QsOperand<kQ4_K> {
+    uint32_t sc[2], mn[2];  // 6-bit scales and mins of sub-blocks 0-3 and 4-7, a byte each
+    uint32_t e;
+    half2 s, m;  // of the block being formed
+    __device__ __forceinline__ void prepare(const QsW<kQ4_K>& w, int) {
+        e = in_vgpr(0x64006400u);
+        sc[0] = w.h.y & 0x3f3f3f3fu;
+        mn[0] = w.h.z & 0x3f3f3f3fu;
+        sc[1] = (w.h.w & 0x0f0f0f0fu) | ((w.h.y >> 2) & 0x30303030u);
+        mn[1] = ((w.h.w >> 4) & 0x0f0f0f0fu) | ((w.h.z >> 2) & 0x30303030u);
+    }
+    __device__ __forceinline__ void get(const QsW<kQ4_K>& w, int, int j, int d, QsOut& o) {
+        if (d == 0) {
+            const uint32_t sel = 0x04000400u | (0x00010001u * static_cast<uint32_t>(j & 3));
+            const half2 t = h2_of(__builtin_amdgcn_perm(0x64646464u, sc[j >> 2], sel));  // 1024 + sc
+            // low nibbles sit under the exponent of 1024 as they are, high ones times 16
+            s = (j & 1) == 0 ? t + h2_all(-1024.0f) : __builtin_elementwise_fma(t, h2_all(0.0625f), h2_all(-64.0f));
+            m = s * h2_all(-1024.0f);
+        }
+        const uint32_t mask = (j & 1) == 0 ? 0x000f000fu : 0x00f000f0u;
+        const uint32_t v = d == 0 ? w.q[j >> 1].x : w.q[j >> 1].y;
+        o.a[2 * d] = u_of(__builtin_elementwise_fma(h2_of((v & mask) | e), s, m));
+        o.a[2 * d + 1] = u_of(__builtin_elementwise_fma(h2_of(((v >> 8) & mask) | e), s, m));
+    }
+};
+template <>
+struct QsOperand<kQ6_K> {
+    uint32_t sc[4];  // scale + 128 of blocks 2 i and 2 i + 1 in bytes 0 and 2
+    uint32_t e1, e2;
+    half2 s1, m1, s2, m2;
+    __device__ __forceinline__ void prepare(const QsW<kQ6_K>& w, int g) {
+        e1 = in_vgpr(0x4c004c00u);
+        e2 = in_vgpr(0x44004400u);
+        const uint32_t v[4] = {w.s.x, w.s.y, w.s.z, w.s.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[i] = (v[i] ^ 0x80808080u) >> (8 * (g >> 1));
+    }
+    __device__ __forceinline__ void get(const QsW<kQ6_K>& w, int, int j, int d, QsOut& o) {
+        const int hf = j >> 2, gr = j & 3;
+        if (d == 0) {
+            const uint32_t sel = (j & 1) == 0 ? 0x04000400u : 0x04020402u;
+            s1 = h2_of(__builtin_amdgcn_perm(0x64646464u, sc[j >> 1], sel)) + h2_all(-1152.0f);
+            m1 = s1 * h2_all(-32.0f);
+            s2 = s1 * h2_all(16.0f);
+            m2 = s1 * h2_all(-80.0f);
+        }
+        const u32x2 lv = w.l[2 * hf + (gr & 1)], uv = w.u[hf];
+        const uint32_t l = d == 0 ? lv.x : lv.y, u = d == 0 ? uv.x : uv.y;
+        // the nibbles of bytes 0, 2 / 1, 3 at bits 6..9 of each half: 16 + l
+        const uint32_t l0 = gr < 2 ? l << 6 : l << 2, l1 = gr < 2 ? l >> 2 : l >> 6;
+        o.a[2 * d] = u_of(__builtin_elementwise_fma(h2_of((l0 & 0x03c003c0u) | e1), s1, m1));
+        o.a[2 * d + 1] = u_of(__builtin_elementwise_fma(h2_of((l1 & 0x03c003c0u) | e1), s1, m1));
+        // the 2-bit values at bits 8, 9: 4 + u
+        const uint32_t u0 = u << (8 - 2 * gr), u1 = u >> (2 * gr);
+        o.b[2 * d] = u_of(__builtin_elementwise_fma(h2_of((u0 & 0x03000300u) | e2), s2, m2));
+        o.b[2 * d + 1] = u_of(__builtin_elementwise_fma(h2_of((u1 & 0x03000300u) | e2), s2, m2));
+    }
+};
+template <>
+struct QsOperand<kQ8_0> {
+    __device__ __forceinline__ void prepare(const QsW<kQ8_0>&, int) {}
+    __device__ __forceinline__ void get(const QsW<kQ8_0>& w, int, int j, int d, QsOut& o) {
+        const uint32_t v = (d == 0 ? w.q[j].x : w.q[j].y) ^ 0x80808080u;  // q + 128 per byte
+        o.a[2 * d] = u_of(h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)) + h2_all(-1152.0f));
+        o.a[2 * d + 1] = u_of(h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)) + h2_all(-1152.0f));
+    }
+};
+template <>
+struct QsOperand<kQ4_0> {
+    __device__ __forceinline__ void prepare(const QsW<kQ4_0>&, int) {}
+    __device__ __forceinline__ void get(const QsW<kQ4_0>& w, int g, int j, int d, QsOut& o) {
+        // values 0-15 are the low nibbles of the 16 bytes, 16-31 the high ones
+        const uint32_t v = (d == 0 ? w.q[j].x : w.q[j].y) >> (4 * (g >> 1));
+        o.a[2 * d] = u_of(h2_of((v & 0x000f000fu) | 0x64006400u) + h2_all(-1032.0f));
+        o.a[2 * d + 1] = u_of(h2_of(((v >> 8) & 0x000f000fu) | 0x64006400u) + h2_all(-1032.0f));
+    }
+};
+__device__ __forceinline__ half8 h8_of(const uint32_t (&v)[4]) {
+    return __builtin_bit_cast(half8, make_uint4(v[0], v[1], v[2], v[3]));
+}
+
+template <int TYPE, int TF>
+__global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     MbMats mats, size_t rbytes, const _Float16* __restrict xq, const float* __restrict dxs,
     const _Float16* __restrict pq, const float* __restrict rscale, int32_t b, int32_t k, int32_t kchunk,
     float* __restrict part, int32_t xmap_tg) {
-    constexpr int WAVES = RT, BM = kQsTok, BN = 32 * RT;
-    static_assert(RT == 8, "one d / s row and one P slice per wave and stage");
+    constexpr int WAVES = 8, BM = 16 * TF, BN = kQsRows, RF = 2;
+    constexpr bool SUPER = TYPE == kQ4_K || TYPE == kQ6_K;  // d per super-block, K of whole super-blocks
+    constexpr int NP = TYPE == kQ6_K ? 2 : 1;               // products per block
+    constexpr int OLD = BN + 4;
+    constexpr int kXHalves = BM * OLD;  // a q stage, or half of the tokens' output rows as floats
     // stage s: q [token][256] with the 16-byte segments of token t at
     // positions c ^ (t % 16) (conflict-free reads of one segment by 16
-    // tokens), d_x / s [block][token], P [token][8 hi, 8 lo]; separate
-    // arrays, so that a load into one stage does not make the compiler wait
-    // before reads of another
-    __shared__ __align__(16) _Float16 xs0[kQsXHalves], xs1[kQsXHalves], xs2[kQsXHalves];
-    __shared__ __align__(16) float sd0[8 * BM], sd1[8 * BM], sd2[8 * BM];
-    __shared__ __align__(16) _Float16 sp0[16 * BM], sp1[16 * BM], sp2[16 * BM];
+    // tokens), d_x / s [token][8] with block j at j ^ (t / 4 % 4), P [token][8
+    // hi, 8 lo] in 8-byte pieces swapped the same way (one piece read by 16
+    // tokens hits distinct banks); separate arrays, so that a load into one
+    // stage does not make the compiler wait before reads of another
+    constexpr int kP = TYPE == kQ4_K ? 16 * BM : 8;
+    constexpr bool S3 = TF < 8;  // three stages (two of 128 tokens fill the LDS)
+    __shared__ __align__(16) _Float16 xs0[kXHalves], xs1[kXHalves], xs2[S3 ? kXHalves : 8];
+    __shared__ __align__(16) float sd0[8 * BM], sd1[8 * BM], sd2[S3 ? 8 * BM : 4];
+    __shared__ __align__(16) _Float16 sp0[kP], sp1[kP], sp2[S3 ? kP : 8];
     __shared__ __align__(16) float srs[BM];
-    __shared__ __align__(16) float sdm[WAVES][2][32];  // per wave: its rows' d and dmin
+    // per wave: its rows' d and dmin, or their d of each block
+    __shared__ __align__(16) float sdm[WAVES][SUPER ? 2 : 8][32];
 
     // the work-group's row group, token group and K range.  Without a split
     // the 1-D grid can be dealt over the XCDs (work-group i runs on XCD i %
@@ -970,24 +637,41 @@ __global__ __launch_bounds__(64 * RT, 1) void matbatch_qs_stream_kernel(
         }
     }
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int li = lane & 31, lh = lane >> 5;
+    const int l16 = lane & 15, lg = lane >> 4;
     const int32_t t0 = by * BM, n0 = (bx - tile0) * BN;
-    const int32_t kb = bz * kchunk;
-    const int32_t nsb = (min(k, kb + kchunk) - kb) / 256;  // super-blocks of the range
-    const int32_t rows_here = min(BM, b - t0);
+    const int32_t kb = bz * kchunk, ke = min(k, kb + kchunk);
+    const int32_t nsb = (ke - kb + 255) / 256;  // super-blocks of the range
+    const int32_t rows_here = min(BM, b - t0), wrows_here = min(BN, n - n0);
 
-    // this lane's weight row, 32 wv + l % 32; rows past N and super-blocks
-    // past the range read zeros (offsets past the resource)
-    const int32_t wrows_here = min(BN, n - n0);
-    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(w + static_cast<size_t>(n0) * rbytes), static_cast<short>(0),
-        wrows_here * static_cast<int32_t>(rbytes), 0x00020000);
+    // this lane's weight rows, 32 wv + 16 f + l % 16; rows past N and
+    // super-blocks past the range read zeros (offsets past the resource,
+    // whose base is the dword at or below the first row)
     constexpr int32_t kWB = QsW<TYPE>::kBytes;
-    const int32_t wbase = (32 * wv + li) * static_cast<int32_t>(rbytes) + (kb / 256) * kWB;
-    using SbRegs = QsW<TYPE>;
-    auto wload = [&](SbRegs& r, int32_t s) { r.load(wrs, s < nsb ? wbase + s * kWB : kMfOob, lh); };
-    // the activations of super-block s into a stage: 4 q loads, one d / s
-    // row and one P slice per wave (token rows past B read zeros)
+    const uint8_t* wt = w + static_cast<size_t>(n0) * rbytes;
+    const int32_t delta = TYPE == kQ4_K ? 0 : static_cast<int32_t>(reinterpret_cast<uintptr_t>(wt) & 3u);
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wt - delta), static_cast<short>(0),
+                                          wrows_here * static_cast<int32_t>(rbytes) + delta, 0x00020000);
+    int32_t wbase[RF];
+#pragma unroll
+    for (int f = 0; f < RF; ++f) {
+        const int32_t row = 32 * wv + 16 * f + l16;
+        wbase[f] = row < wrows_here ? row * static_cast<int32_t>(rbytes) + delta + kb / 256 * kWB : kMfOob / 2;
+    }
+    struct SbRegs {
+        QsW<TYPE> f[RF];
+    };
+    SbRegs R;
+    // part P of super-block s
+    auto wload = [&]<int P>(std::integral_constant<int, P>, int32_t s) {
+        const int32_t nblk = SUPER ? 8 : (ke - kb - 256 * s) / 32, at = s < nsb ? s * kWB : kMfOob / 2;
+#pragma unroll
+        for (int f = 0; f < RF; ++f) R.f[f].template load<P>(wrs, wbase[f] + at, lg, nblk);
+    };
+    // the activations of super-block s into a stage (token rows past B and
+    // values past K read zeros); with fewer than 64 tokens some waves load
+    // the same d / s and P pieces again, so that every wave issues kXLoads
+    constexpr int kXQ = TF, kXP = TF > 4 ? TF / 4 : 1;  // q loads, d / s and P loads per wave
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<_Float16*>(xq + static_cast<size_t>(t0) * k), static_cast<short>(0),
         rows_here * k * static_cast<int32_t>(sizeof(_Float16)), 0x00020000);
@@ -998,287 +682,302 @@ __global__ __launch_bounds__(64 * RT, 1) void matbatch_qs_stream_kernel(
         const_cast<_Float16*>(TYPE == kQ4_K ? pq + static_cast<size_t>(t0) * (k / 256) * 16 : xq), static_cast<short>(0),
         TYPE == kQ4_K ? rows_here * (k / 256) * 16 * static_cast<int32_t>(sizeof(_Float16)) : 0, 0x00020000);
     auto xload = [&](_Float16* xst, float* sdt, _Float16* spt, int32_t s) {
-        const bool in = s < nsb;
-        const int32_t k0 = kb + 256 * s;
+        // a wave's loads differ by a wave-uniform distance (16 or 64 tokens);
+        // the lane's offsets are hidden from the compiler, which would
+        // otherwise keep a register for each load across the loop
+        const int32_t k0 = kb + 256 * s, past = s < nsb ? 0 : kMfOob;
+        const int tq = 2 * wv + (lane >> 5), c = (lane & 31) ^ (tq & 15);  // token rows 2 wv, 2 wv + 1 (+ 16 i)
+        int32_t vq = (tq * k + 8 * c) * 2;
+        const int pw = TF >= 4 ? wv : wv % (2 * TF);
+        // tokens 8 pw .. (+ 64 i); the swizzles of d_x / s and P
+        const int tp = 8 * pw + (lane >> 3), sw = (tp >> 2) & 3, blk = (lane & 7) ^ sw;
+        int32_t vd = (tp * (k / 32) + blk) * 4, vp = (tp * (k / 256) * 16 + 2 * ((lane & 7) ^ (2 * sw))) * 2;
+        if constexpr (!SUPER) {
+            vq = k0 + 8 * c < ke ? vq : kMfOob / 2;
+            vd = k0 + 32 * blk < ke ? vd : kMfOob / 2;
+        }
+        asm volatile("" : "+v"(vq), "+v"(vd), "+v"(vp));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int q = i * WAVES + wv;  // token rows 2 q, 2 q + 1
-            const int t = 2 * q + (lane >> 5), c = (lane & 31) ^ (t & 15);
-            const int32_t off = in ? (t * k + k0 + 8 * c) * static_cast<int32_t>(sizeof(_Float16)) : kMfOob;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr)(xst + 512 * q), 16, off, 0, 0, 0);
+        for (int i = 0; i < kXQ; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr)(xst + 512 * (i * WAVES + wv)), 16,
+                                                     vq + (past ? kMfOob / 2 : (16 * i * k + k0) * 2), 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kXP; ++i) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(drs, (lds_ptr)(sdt + 64 * (8 * i + pw)), 4,
+                                                     vd + (past ? kMfOob / 2 : (64 * i * (k / 32) + k0 / 32) * 4), 0, 0,
+                                                     0);
+            if constexpr (TYPE == kQ4_K)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    prs, (lds_ptr)(spt + 128 * (8 * i + pw)), 4,
+                    vp + (past ? kMfOob / 2 : (64 * i * (k / 256) + k0 / 256) * 32), 0, 0, 0);
         }
-        {
-            const int32_t off = in ? (lane * (k / 32) + k0 / 32 + wv) * static_cast<int32_t>(sizeof(float)) : kMfOob;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(drs, (lds_ptr)(sdt + 64 * wv), 4, off, 0, 0, 0);
-        }
+    };
+    constexpr int kXLoads = kXQ + kXP * (TYPE == kQ4_K ? 2 : 1);
+    // the loads that may be in flight past a super-block's barrier: its own
+    // (weights of the next one and, with three stages, activations two ahead)
+    constexpr int kLoads = RF * QsW<TYPE>::kLoads + (S3 ? kXLoads : 0);
+    auto wfirst = [&] {
+        [&]<int... P>(std::integer_sequence<int, P...>) {
+            (wload(std::integral_constant<int, P - 1>{}, 0), ...);
+        }(std::make_integer_sequence<int, 9>{});
+    };
+    // up to 64 tokens the weights first, which come from farthest away, and
+    // the row scales before them, without a branch, so that their wait covers
+    // nothing else (the 128-token kernel spills 10 registers in this order:
+    // 8% slower)
+    if constexpr (S3) {
+        const float rsv = rscale[t0 + min(tid, rows_here - 1)];
+        wfirst();
+        xload(xs0, sd0, sp0, 0);
+        xload(xs1, sd1, sp1, 1);
+        if (tid < BM) srs[tid] = rsv;
+        step_barrier<kXLoads>();
+    } else {
+        if (tid < BM) srs[tid] = rscale[t0 + min(tid, rows_here - 1)];
+        xload(xs0, sd0, sp0, 0);
+        wfirst();
+        step_barrier<kLoads>();
+    }
+
+    floatx4 acc[RF][TF], S[RF][TF];
+#pragma unroll
+    for (int f = 0; f < RF; ++f)
+#pragma unroll
+        for (int t = 0; t < TF; ++t) acc[f][t] = S[f][t] = floatx4{};
+
+    // super-block s from its registers and stage, the next one's weights
+    // loaded as the registers fall free
+    auto process = [&](const _Float16* xst, const float* sdt, const _Float16* spt, int32_t s) {
+        QsOperand<TYPE> op[RF];
+#pragma unroll
+        for (int f = 0; f < RF; ++f) op[f].prepare(R.f[f], lg);
+        // the accumulator rows' scales, exchanged through LDS within the wave
         if constexpr (TYPE == kQ4_K) {
-            const int dw = 64 * wv + lane, t = dw >> 3;
-            const int32_t off =
-                in ? ((t * (k / 256) + k0 / 256) * 16 + 2 * (dw & 7)) * static_cast<int32_t>(sizeof(_Float16)) : kMfOob;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (lds_ptr)(spt + 128 * wv), 4, off, 0, 0, 0);
-        }
-    };
-    // activation loads per wave and super-block (q; d / s; Q4_K: P)
-    constexpr int kXLoads = TYPE == kQ4_K ? 6 : 5;
-    if (tid < BM) srs[tid] = tid < rows_here ? rscale[t0 + tid] : 0.0f;
-    SbRegs R0, R1;
-    wload(R0, 0);
-    xload(xs0, sd0, sp0, 0);
-    xload(xs1, sd1, sp1, 1);
-    step_barrier<kXLoads>();
-
-    floatx16 acc[2], S[2];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[tt][r] = S[tt][r] = 0.0f;
-
-    // one Q4_K super-block from its registers and stage
-    auto process_q4k = [&](const QsW<kQ4_K>& R, const _Float16* xst, const float* sdt, const _Float16* spt) {
-        if (lh == 0) {
-            sdm[wv][0][li] = half_bits_to_float(R.h.x & 0xffffu);
-            sdm[wv][1][li] = half_bits_to_float(R.h.x >> 16);
-        }
-        int sc[8], mn[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) k4_scale_min(j, R.h.y, R.h.z, R.h.w, sc[j], mn[j]);
-        const uint32_t qd[4][4] = {{R.q[0].x, R.q[0].y, R.q[0].z, R.q[0].w},
-                                   {R.q[1].x, R.q[1].y, R.q[1].z, R.q[1].w},
-                                   {R.q[2].x, R.q[2].y, R.q[2].z, R.q[2].w},
-                                   {R.q[3].x, R.q[3].y, R.q[3].z, R.q[3].w}};
-        // block j's operands: activations of both token tiles and K slices,
-        // their block scales, and the weights as sc q, two codes per
-        // instruction: a byte permute puts codes a and c under the exponent
-        // of 1024 (fp16 bits 0x6400 | a are 1024 + a), and one packed fma
-        // gives (1024 + a) sc - 1024 sc = a sc with a single rounding of an
-        // exact value (a sc <= 945)
-        auto operands = [&](int j, half8 (&xo)[2][2], float (&dvv)[2], half8 (&wq)[2]) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int tr = 32 * tt + li;
-#pragma unroll
-                for (int sl = 0; sl < 2; ++sl) {
-                    const int c = (4 * j + 2 * lh + sl) ^ (tr & 15);
-                    xo[tt][sl] = *reinterpret_cast<const half8*>(&xst[256 * tr + 8 * c]);
-                }
-                dvv[tt] = sdt[64 * j + tr];
+            if (lg < 2) {
+                const uint32_t h = lg == 0 ? R.f[0].h.x : R.f[1].h.x;
+                sdm[wv][0][16 * lg + l16] = half_bits_to_float(h & 0xffffu);
+                sdm[wv][1][16 * lg + l16] = half_bits_to_float(h >> 16);
             }
-            const _Float16 scf = static_cast<_Float16>(static_cast<float>(sc[j]));
-            const _Float16 off = static_cast<_Float16>(-1024.0f * static_cast<float>(sc[j]));
-            const half2 s2 = {scf, scf}, m2 = {off, off};
-            uint32_t o[8];
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const uint32_t x = (qd[j >> 1][d] >> (4 * (j & 1))) & 0x0f0f0f0fu;
-                const half2 p0 = __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, x, 0x04010400u));
-                const half2 p1 = __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u));
-                o[2 * d] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(p0, s2, m2));
-                o[2 * d + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(p1, s2, m2));
-            }
-            wq[0] = __builtin_bit_cast(half8, make_uint4(o[0], o[1], o[2], o[3]));
-            wq[1] = __builtin_bit_cast(half8, make_uint4(o[4], o[5], o[6], o[7]));
-        };
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            half8 xo[2][2], wq[2];
-            float dvv[2];
-            operands(j, xo, dvv, wq);
-            floatx16 blk[2];
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const floatx16 zero = {};
-                blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[0], xo[tt][0], zero, 0, 0, 0);
-                blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[1], xo[tt][1], blk[tt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) S[tt][r] = j == 0 ? dvv[tt] * blk[tt][r] : fmaf(dvv[tt], blk[tt][r], S[tt][r]);
-        }
-        // acc += d S - dmin (m . P); the mins of sub-blocks 4 h .. + 3 are
-        // the min product's A operand (K = the super-block's 8 sub-blocks)
-        half4 mn4;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) mn4[q] = static_cast<_Float16>(static_cast<float>(lh ? mn[4 + q] : mn[q]));
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int tr = 32 * tt + li;
-            const half4 ph = *reinterpret_cast<const half4*>(&spt[16 * tr + 4 * lh]);
-            const half4 pl = *reinterpret_cast<const half4*>(&spt[16 * tr + 8 + 4 * lh]);
-            const floatx16 zero = {};
-            floatx16 M = __builtin_amdgcn_mfma_f32_32x32x8f16(mn4, ph, zero, 0, 0, 0);
-            M = __builtin_amdgcn_mfma_f32_32x32x8f16(mn4, pl, M, 0, 0, 0);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 d4 = *reinterpret_cast<const float4*>(&sdm[wv][0][8 * g + 4 * lh]);
-                const float4 m4 = *reinterpret_cast<const float4*>(&sdm[wv][1][8 * g + 4 * lh]);
-                const float dq[4] = {d4.x, d4.y, d4.z, d4.w}, mq[4] = {m4.x, m4.y, m4.z, m4.w};
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int r = 4 * g + q;
-                    acc[tt][r] = fmaf(S[tt][r], dq[q], acc[tt][r]);
-                    acc[tt][r] = fmaf(M[r], -mq[q], acc[tt][r]);
-                }
-            }
-        }
-    };
-
-    // one Q6_K super-block (index sidx of the range) from its registers and stage
-    auto process_q6k = [&](const QsW<kQ6_K>& R, const _Float16* xst, const float* sdt, int32_t sidx) {
-        // pieces realigned as they are used (blocks are 2-byte aligned: the shift is 0 or 2)
-        const int sh = (wbase + sidx * kWB) & 3;
-        auto piece = [&](int i, int d) {
-            const uint32_t lo = d == 0 ? R.p[i].x : d == 1 ? R.p[i].y : d == 2 ? R.p[i].z : R.p[i].w;
-            const uint32_t hi = d == 0 ? R.p[i].y : d == 1 ? R.p[i].z : d == 2 ? R.p[i].w : R.e[i];
-            return __builtin_amdgcn_alignbyte(hi, lo, sh);
-        };
-        if (lh == 0) sdm[wv][0][li] = half_bits_to_float((R.e[6] >> (8 * sh)) & 0xffffu);
-        // the lane's scales: group g of half hf uses byte 8 hf + 2 g + h of the 16
-        int sc[2][4];
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const uint32_t wd = piece(6, 2 * hf + (g >> 1));
-                sc[hf][g] = static_cast<int>(static_cast<int8_t>((wd >> (8 * (2 * (g & 1) + lh))) & 0xffu));
-            }
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int jb = 4 * hf + g;  // the 32-value block of the super-block
-                half8 xo[2][2];
-                float dvv[2];
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const int tr = 32 * tt + li;
-#pragma unroll
-                    for (int sl = 0; sl < 2; ++sl) {
-                        const int c = (4 * jb + 2 * lh + sl) ^ (tr & 15);
-                        xo[tt][sl] = *reinterpret_cast<const half8*>(&xst[256 * tr + 8 * c]);
-                    }
-                    dvv[tt] = sdt[64 * jb + tr];
-                }
-                // sc (q - 32) = sc (l - 16) + 16 sc (u - 1) with q = l + 16 u
-                // (l the ql nibble, u the qh pair): |sc (l - 16)| <= 2048 and
-                // 16 sc (u - 1) = 16 x an integer of at most 256, both exact in
-                // fp16 for every int8 scale; from the fp16 integers 1024 + l and
-                // 1024 + u, one exact add and one exact multiply each
-                const _Float16 scf = static_cast<_Float16>(static_cast<float>(sc[hf][g]));
-                const _Float16 sc16 = static_cast<_Float16>(16.0f * static_cast<float>(sc[hf][g]));
-                const half2 s1 = {scf, scf}, s2 = {sc16, sc16};
-                const half2 o1 = {static_cast<_Float16>(-1040.0f), static_cast<_Float16>(-1040.0f)};
-                const half2 o2 = {static_cast<_Float16>(-1025.0f), static_cast<_Float16>(-1025.0f)};
-                uint32_t a1[8], a2[8];
-#pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const uint32_t l4 = (piece(2 * hf + (g & 1), d) >> (4 * (g >> 1))) & 0x0f0f0f0fu;
-                    const uint32_t u4 = (piece(4 + hf, d) >> (2 * g)) & 0x03030303u;
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const uint32_t sel = e == 0 ? 0x04010400u : 0x04030402u;
-                        const half2 pl = __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, l4, sel));
-                        const half2 pu = __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, u4, sel));
-                        a1[2 * d + e] = __builtin_bit_cast(uint32_t, (pl + o1) * s1);
-                        a2[2 * d + e] = __builtin_bit_cast(uint32_t, (pu + o2) * s2);
-                    }
-                }
-                const half8 w10 = __builtin_bit_cast(half8, make_uint4(a1[0], a1[1], a1[2], a1[3]));
-                const half8 w11 = __builtin_bit_cast(half8, make_uint4(a1[4], a1[5], a1[6], a1[7]));
-                const half8 w20 = __builtin_bit_cast(half8, make_uint4(a2[0], a2[1], a2[2], a2[3]));
-                const half8 w21 = __builtin_bit_cast(half8, make_uint4(a2[4], a2[5], a2[6], a2[7]));
-                floatx16 blk[2];
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const floatx16 zero = {};
-                    blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w10, xo[tt][0], zero, 0, 0, 0);
-                    blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w11, xo[tt][1], blk[tt], 0, 0, 0);
-                    blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w20, xo[tt][0], blk[tt], 0, 0, 0);
-                    blk[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w21, xo[tt][1], blk[tt], 0, 0, 0);
-                }
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        S[tt][r] = jb == 0 ? dvv[tt] * blk[tt][r] : fmaf(dvv[tt], blk[tt][r], S[tt][r]);
-            }
-        // acc += d S (d of the accumulator's rows, from the wave's exchange slots)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 d4 = *reinterpret_cast<const float4*>(&sdm[wv][0][8 * g + 4 * lh]);
-                acc[tt][4 * g] = fmaf(S[tt][4 * g], d4.x, acc[tt][4 * g]);
-                acc[tt][4 * g + 1] = fmaf(S[tt][4 * g + 1], d4.y, acc[tt][4 * g + 1]);
-                acc[tt][4 * g + 2] = fmaf(S[tt][4 * g + 2], d4.z, acc[tt][4 * g + 2]);
-                acc[tt][4 * g + 3] = fmaf(S[tt][4 * g + 3], d4.w, acc[tt][4 * g + 3]);
-            }
-    };
-    auto process = [&](const SbRegs& R, const _Float16* xst, const float* sdt, const _Float16* spt, int32_t sidx) {
-        if constexpr (TYPE == kQ4_K) {
-            (void)sidx;
-            process_q4k(R, xst, sdt, spt);
+        } else if constexpr (TYPE == kQ6_K) {
+            if (lg < 2) sdm[wv][0][16 * lg + l16] = half_bits_to_float(lg == 0 ? R.f[0].d : R.f[1].d);
         } else {
-            (void)spt;
-            process_q6k(R, xst, sdt, sidx);
+#pragma unroll
+            for (int f = 0; f < RF; ++f)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) sdm[wv][2 * lg + e][16 * f + l16] = half_bits_to_float(R.f[f].d[e]);
+        }
+        wload(std::integral_constant<int, -1>{}, s + 1);
+        // LDS offsets; hidden from the compiler, which would otherwise keep
+        // one register per block for each across the loop
+        int xa = 256 * l16 + 8 * (lg ^ l16), da = 8 * l16 + (l16 >> 2);
+        asm volatile("" : "+v"(xa), "+v"(da));
+        auto x_at = [&](int j, int t) {
+            return *reinterpret_cast<const half8*>(&xst[(xa ^ (32 * j)) + 4096 * t]);
+        };
+        auto dx_at = [&](int j, int t) { return sdt[(da ^ j) + 128 * t]; };
+        QsOut wq[2][RF];
+        floatx4 dr[2][RF];
+        auto dr_at = [&](int j, int f) { return *reinterpret_cast<const floatx4*>(&sdm[wv][SUPER ? 0 : j][16 * f + 4 * lg]); };
+        auto mul = [&](const QsOut& o, const half8& x) {
+            floatx4 v = __builtin_amdgcn_mfma_f32_16x16x32_f16(h8_of(o.a), x, floatx4{}, 0, 0, 0);
+            if constexpr (NP == 2) v = __builtin_amdgcn_mfma_f32_16x16x32_f16(h8_of(o.b), x, v, 0, 0, 0);
+            return v;
+        };
+        auto scale = [&](int j, int f, int t, float dx, const floatx4& v) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float c = SUPER ? dx : dx * dr[j & 1][f][r];
+                S[f][t][r] = j == 0 ? c * v[r] : fmaf(c, v[r], S[f][t][r]);
+            }
+        };
+#pragma unroll
+        for (int f = 0; f < RF; ++f) {
+            op[f].get(R.f[f], lg, 0, 0, wq[0][f]);
+            op[f].get(R.f[f], lg, 0, 1, wq[0][f]);
+            if constexpr (!SUPER) dr[0][f] = dr_at(0, f);
+        }
+        if constexpr (TF >= 4) {
+            // One region per block and token tile: a region multiplies its
+            // tile, scales the tile of the region before it, reads the
+            // activations kAhead regions ahead and forms its share of the
+            // next block's weights (a quarter every TF / 4 regions).  The
+            // scheduling barriers keep that order (left alone, the compiler
+            // reads and forms far ahead and spills).
+            constexpr int kAhead = TYPE == kQ4_K ? 4 : 2, NX = kAhead + 1;
+            half8 xo[NX];
+            float dx[NX];
+            floatx4 blk[2][RF];
+            auto read = [&](int rg) {
+                xo[rg % NX] = x_at(rg / TF, rg % TF);
+                dx[rg % NX] = dx_at(rg / TF, rg % TF);
+            };
+            float dxp = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) read(i);
+            auto region = [&]<int rg>(std::integral_constant<int, rg>) {
+                constexpr int j = rg / TF, t = rg % TF, q = t * 4 / TF;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int f = 0; f < RF; ++f) blk[rg & 1][f] = mul(wq[j & 1][f], xo[rg % NX]);
+                __builtin_amdgcn_sched_barrier(0);  // products first: their results rest until the next region
+                if constexpr (rg > 0) {
+#pragma unroll
+                    for (int f = 0; f < RF; ++f) scale((rg - 1) / TF, f, (rg - 1) % TF, dxp, blk[(rg - 1) & 1][f]);
+                }
+                dxp = dx[rg % NX];
+                if constexpr (rg + kAhead < 8 * TF) read(rg + kAhead);
+                if constexpr (t == 0) wload(std::integral_constant<int, j>{}, s + 1);
+                if constexpr (j < 7 && t % (TF / 4) == 0) {
+                    op[q >> 1].get(R.f[q >> 1], lg, j + 1, q & 1, wq[(j + 1) & 1][q >> 1]);
+                    if constexpr (!SUPER && q == 3) {
+#pragma unroll
+                        for (int f = 0; f < RF; ++f) dr[(j + 1) & 1][f] = dr_at(j + 1, f);
+                    }
+                }
+            };
+            [&]<int... G>(std::integer_sequence<int, G...>) {
+                (region(std::integral_constant<int, G>{}), ...);
+            }(std::make_integer_sequence<int, 8 * TF>{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int f = 0; f < RF; ++f) scale(7, f, TF - 1, dxp, blk[1][f]);
+        } else {
+            auto block = [&]<int j>(std::integral_constant<int, j>) {
+                __builtin_amdgcn_sched_barrier(0);
+                floatx4 blk[RF][TF];
+                float dx[TF];
+#pragma unroll
+                for (int t = 0; t < TF; ++t) {
+                    const half8 xo = x_at(j, t);
+                    dx[t] = dx_at(j, t);
+#pragma unroll
+                    for (int f = 0; f < RF; ++f) blk[f][t] = mul(wq[j & 1][f], xo);
+                }
+                wload(std::integral_constant<int, j>{}, s + 1);
+                if constexpr (j < 7) {
+#pragma unroll
+                    for (int f = 0; f < RF; ++f) {
+                        op[f].get(R.f[f], lg, j + 1, 0, wq[(j + 1) & 1][f]);
+                        op[f].get(R.f[f], lg, j + 1, 1, wq[(j + 1) & 1][f]);
+                        if constexpr (!SUPER) dr[(j + 1) & 1][f] = dr_at(j + 1, f);
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < TF; ++t)
+#pragma unroll
+                    for (int f = 0; f < RF; ++f) scale(j, f, t, dx[t], blk[f][t]);
+            };
+            [&]<int... J>(std::integer_sequence<int, J...>) {
+                (block(std::integral_constant<int, J>{}), ...);
+            }(std::make_integer_sequence<int, 8>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (TYPE == kQ4_K) {
+            // acc += d S - dmin (m . P): the mins of sub-blocks 4 (g % 2) .. + 3
+            // against P hi (g < 2) and P lo, K = 16 in one product
+            half4 mo[RF];
+#pragma unroll
+            for (int f = 0; f < RF; ++f) {
+                const uint32_t m = (lg & 1) != 0 ? op[f].mn[1] : op[f].mn[0];
+                const half2 a = h2_of(__builtin_amdgcn_perm(0x64646464u, m, 0x04010400u)) + h2_all(-1024.0f);
+                const half2 c = h2_of(__builtin_amdgcn_perm(0x64646464u, m, 0x04030402u)) + h2_all(-1024.0f);
+                mo[f] = __builtin_shufflevector(a, c, 0, 1, 2, 3);
+            }
+#pragma unroll
+            for (int f = 0; f < RF; ++f) {
+                const floatx4 d = *reinterpret_cast<const floatx4*>(&sdm[wv][0][16 * f + 4 * lg]);
+                const floatx4 dm = *reinterpret_cast<const floatx4*>(&sdm[wv][1][16 * f + 4 * lg]);
+#pragma unroll
+                for (int t = 0; t < TF; ++t) {
+                    const half4 po = *reinterpret_cast<const half4*>(&spt[16 * (16 * t + l16) + 4 * (lg ^ (l16 >> 2))]);
+                    const floatx4 M = __builtin_amdgcn_mfma_f32_16x16x16f16(mo[f], po, floatx4{}, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[f][t][r] = fmaf(S[f][t][r], d[r], acc[f][t][r]);
+                        acc[f][t][r] = fmaf(M[r], -dm[r], acc[f][t][r]);
+                    }
+                }
+            }
+        } else if constexpr (TYPE == kQ6_K) {
+#pragma unroll
+            for (int f = 0; f < RF; ++f) {
+                const floatx4 d = *reinterpret_cast<const floatx4*>(&sdm[wv][0][16 * f + 4 * lg]);
+#pragma unroll
+                for (int t = 0; t < TF; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[f][t][r] = fmaf(S[f][t][r], d[r], acc[f][t][r]);
+            }
+        } else {
+#pragma unroll
+            for (int f = 0; f < RF; ++f)
+#pragma unroll
+                for (int t = 0; t < TF; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[f][t][r] += S[f][t][r];
         }
     };
 
-    // super-block s in register set s % 2 and stage s % 3: each starts
-    // the loads of the next super-block's weights and of the activations two
-    // ahead (into the stage the one before it left), and ends with the
-    // barrier after which the next is in place for every wave (only the
-    // activations two ahead may still be in flight) and its own stage may be
-    // refilled
-#define GNCX_QS_STEP(RA, RB, XA, DA, PA, XC, DC, PC, OFF) \
-    wload(RB, s + (OFF) + 1);                        \
-    xload(XC, DC, PC, s + (OFF) + 2);                \
-    process(RA, XA, DA, PA, s + (OFF));              \
-    step_barrier<kXLoads>();                         \
+    // super-block s in stage s % 3 (% 2): each starts the loads of the
+    // activations two (one) ahead, into the stage the one before it left, and
+    // ends with the barrier after which the next stage is in place for every
+    // wave and its own may be refilled
+#define GNCX_QS_STEP(XA, DA, PA, XC, DC, PC, OFF) \
+    xload(XC, DC, PC, s + (OFF) + (S3 ? 2 : 1));  \
+    process(XA, DA, PA, s + (OFF));               \
+    step_barrier<kLoads>();                       \
     if (s + (OFF) + 1 >= nsb) break;
-    for (int32_t s = 0; s < nsb; s += 6) {
-        GNCX_QS_STEP(R0, R1, xs0, sd0, sp0, xs2, sd2, sp2, 0)
-        GNCX_QS_STEP(R1, R0, xs1, sd1, sp1, xs0, sd0, sp0, 1)
-        GNCX_QS_STEP(R0, R1, xs2, sd2, sp2, xs1, sd1, sp1, 2)
-        GNCX_QS_STEP(R1, R0, xs0, sd0, sp0, xs2, sd2, sp2, 3)
-        GNCX_QS_STEP(R0, R1, xs1, sd1, sp1, xs0, sd0, sp0, 4)
-        GNCX_QS_STEP(R1, R0, xs2, sd2, sp2, xs1, sd1, sp1, 5)
+    if constexpr (S3) {
+        for (int32_t s = 0; s < nsb; s += 3) {
+            GNCX_QS_STEP(xs0, sd0, sp0, xs2, sd2, sp2, 0)
+            GNCX_QS_STEP(xs1, sd1, sp1, xs0, sd0, sp0, 1)
+            GNCX_QS_STEP(xs2, sd2, sp2, xs1, sd1, sp1, 2)
+        }
+    } else {
+        for (int32_t s = 0; s < nsb; s += 2) {
+            GNCX_QS_STEP(xs0, sd0, sp0, xs1, sd1, sp1, 0)
+            GNCX_QS_STEP(xs1, sd1, sp1, xs0, sd0, sp0, 1)
+        }
     }
 #undef GNCX_QS_STEP
 
-    // the tile of token tile tt in stage tt's q array as [32 tokens][BN + 4]
-    // floats (rows padded: conflict-free), then whole token rows out
-    constexpr int OLD = BN + 4;
-    static_assert(32 * OLD * 2 <= kQsXHalves, "an output tile fits in a stage");
+    // the tile as [token][BN + 4] floats in LDS, then whole token rows out
     __syncthreads();
+    constexpr int HT = BM / 2;  // tokens per stage array
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        float* ost = reinterpret_cast<float*>(tt == 0 ? xs0 : xs1);
-        const float rs = srs[32 * tt + li];
+    for (int t = 0; t < TF; ++t) {
+        const int tok = 16 * t + l16;
+        float* ost = reinterpret_cast<float*>(tok < HT ? xs0 : xs1) + (tok % HT) * OLD;
+        const float rs = srs[tok];
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<float4*>(&ost[li * OLD + 32 * wv + 8 * g + 4 * lh]) =
-                make_float4(acc[tt][4 * g] * rs, acc[tt][4 * g + 1] * rs, acc[tt][4 * g + 2] * rs,
-                            acc[tt][4 * g + 3] * rs);
+        for (int f = 0; f < RF; ++f)
+            *reinterpret_cast<floatx4*>(&ost[32 * wv + 16 * f + 4 * lg]) = acc[f][t] * rs;
     }
     __syncthreads();
     float* dst = gridDim.z > 1 ? part + (static_cast<size_t>(bz) * mats.ntot + npre) * b : y;
-    const int32_t rows = min(BN, n - n0);
     if ((n & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-        // 4 rows per lane, BN / 4 lanes per token
-        constexpr int LPT = BN / 4, TPI = 64 * WAVES / LPT;
-        const int c = 4 * (tid % LPT);
-        for (int tl = tid / LPT; tl < rows_here; tl += TPI) {
-            const float* ost = reinterpret_cast<const float*>(tl < 32 ? xs0 : xs1);
-            if (c < rows)
-                *reinterpret_cast<float4*>(&dst[static_cast<size_t>(t0 + tl) * n + n0 + c]) =
-                    *reinterpret_cast<const float4*>(&ost[(tl & 31) * OLD + c]);
+        // 4 rows per lane, one token per wave and step
+        const int c = 4 * lane;
+        for (int t = wv; t < rows_here; t += WAVES) {
+            const float* ost = reinterpret_cast<const float*>(t < HT ? xs0 : xs1) + (t % HT) * OLD;
+            if (c < wrows_here)
+                *reinterpret_cast<floatx4*>(&dst[static_cast<size_t>(t0 + t) * n + n0 + c]) =
+                    *reinterpret_cast<const floatx4*>(&ost[c]);
+        }
+    } else if ((n & 1) == 0 && (reinterpret_cast<uintptr_t>(dst) & 7u) == 0) {
+        const int c = 2 * (tid & 127);
+#pragma unroll 4
+        for (int t = tid >> 7; t < rows_here; t += 4) {
+            const float* ost = reinterpret_cast<const float*>(t < HT ? xs0 : xs1) + (t % HT) * OLD;
+            if (c < wrows_here)
+                *reinterpret_cast<float2*>(&dst[static_cast<size_t>(t0 + t) * n + n0 + c]) =
+                    *reinterpret_cast<const float2*>(&ost[c]);
         }
     } else {
-        for (int e = tid; e < rows_here * BN; e += 64 * WAVES) {
-            const int tl = e / BN, c = e % BN;
-            const float* ost = reinterpret_cast<const float*>(tl < 32 ? xs0 : xs1);
-            if (c < rows) dst[static_cast<size_t>(t0 + tl) * n + n0 + c] = ost[(tl & 31) * OLD + c];
+        const int c = tid & 255;
+#pragma unroll 4
+        for (int t = tid >> 8; t < rows_here; t += 2) {
+            const float* ost = reinterpret_cast<const float*>(t < HT ? xs0 : xs1) + (t % HT) * OLD;
+            if (c < wrows_here) dst[static_cast<size_t>(t0 + t) * n + n0 + c] = ost[c];
         }
     }
 }
@@ -1308,7 +1007,6 @@ __global__ __launch_bounds__(64 * RT, 1) void matbatch_qs_stream_kernel(
 // 4096, B = 2048).
 constexpr int kBfKs = 128;  // K per stage
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // bf16 parts of 8 values: truncated top 16 bits, the remainder again, and the
 // rest (exact: at most 8 significant bits are left).  Infinite or NaN values
@@ -1544,134 +1242,51 @@ __global__ __launch_bounds__(512, 1) void matbatch_bf16_kernel(const uint8_t* __
 // load-then-add waited on memory once per range).
 constexpr int kRedU = 16;
 
+// V: float, or floatx4 where every output is whole, aligned groups of four
+// (64 x 4096 outputs of 16 ranges: see launch_reduce)
+template <class V>
 __global__ __launch_bounds__(kThreads) void matbatch_reduce_kernel(const float* __restrict part, int32_t splits,
                                                                    RedMats r) {
-    const size_t count = r.end[r.count - 1];
+    constexpr size_t W = sizeof(V) / sizeof(float);
+    const size_t count = r.end[r.count - 1] / W;
+    const V* __restrict p = reinterpret_cast<const V*>(part);
     for (size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x; i < count;
          i += static_cast<size_t>(gridDim.x) * kThreads) {
-        float v[kRedU];
+        V v[kRedU];
 #pragma unroll
-        for (int u = 0; u < kRedU; ++u) v[u] = u < splits ? part[static_cast<size_t>(u) * count + i] : 0.0f;
-        float acc = v[0];
+        for (int u = 0; u < kRedU; ++u) v[u] = u < splits ? p[static_cast<size_t>(u) * count + i] : V{};
+        V acc = v[0];
 #pragma unroll
         for (int u = 1; u < kRedU; ++u)
             if (u < splits) acc += v[u];
-        for (int32_t z = kRedU; z < splits; ++z) acc += part[static_cast<size_t>(z) * count + i];
+        for (int32_t z = kRedU; z < splits; ++z) acc += p[static_cast<size_t>(z) * count + i];
         float* y = r.y[0];
         size_t first = 0;
 #pragma unroll
         for (int m = 1; m < kMaxMbMats; ++m) {
-            if (r.count > m && i >= r.end[m - 1]) {
+            if (r.count > m && i * W >= r.end[m - 1]) {
                 y = r.y[m];
                 first = r.end[m - 1];
             }
         }
-        y[i - first] = acc;
+        *reinterpret_cast<V*>(&y[i * W - first]) = acc;
     }
 }
 
 hipError_t launch_reduce(const float* part, int32_t splits, const RedMats& r, hipStream_t stream) {
-    size_t g = (r.end[r.count - 1] + kThreads - 1) / kThreads;
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(matbatch_reduce_kernel, dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, stream, part,
-                       splits, r);
+    bool four = (reinterpret_cast<uintptr_t>(part) & 15u) == 0;
+    for (int32_t i = 0; i < r.count; ++i)
+        four = four && r.end[i] % 4 == 0 && (reinterpret_cast<uintptr_t>(r.y[i]) & 15u) == 0;
+    const size_t count = r.end[r.count - 1] / (four ? 4 : 1);
+    const size_t g = std::min<size_t>((count + kThreads - 1) / kThreads, 4096);
+    if (four)
+        hipLaunchKernelGGL(matbatch_reduce_kernel<floatx4>, dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, stream,
+                           part, splits, r);
+    else
+        hipLaunchKernelGGL(matbatch_reduce_kernel<float>, dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, stream,
+                           part, splits, r);
     return hipGetLastError();
 }
-
-struct MfmaPlan {
-    int wm, wn;
-    int32_t splits, kchunk;
-    int mw = 2;  // waves along the tokens (4: 512-thread work-groups)
-};
-
-// From 129 tokens, 256-token tiles of 8 waves (one work-group per CU, 111 KB
-// of LDS): 256 x 128 when that gives at least 192 tiles, else 256 x 64 when
-// that does, else 256 x 128 with K split until about 256 work-groups run.
-// Twice the tokens per dequantised weight step, with the dequantising waves
-// and MFMA-only waves sharing each SIMD, measured 1.1-1.4x the 128 x 128 tile
-// (Q4_K 4096 x 14336 at B = 512: 111 vs 141 us; 4096 x 4096 at B = 2048: 116
-// vs 149 us) with bit-identical results (same K order); with K split, Q6_K
-// 14336 -> 4096 at B = 200 / 256 / 512 took 139 / 144 / 258 us against 266 /
-// 268 / 480 us for 64 x 64 tiles with K split.  From 65 to 128 tokens,
-// 128 x 128 tiles of 4 waves with K split until about 512 work-groups run
-// (Q6_K 14336 -> 4096 at B = 128: 108 against 157 us).  Up to 64 tokens, the
-// largest tile whose grid fills every CU with as many work-groups as its LDS
-// lets one CU hold (2 for 128 x 128 and 128 x 64, 4 for 64 x 64), else 64 x 64
-// tiles with K split until it does (ranges of at least 256).
-MfmaPlan mfma_plan(int32_t b, int32_t k, int32_t n) {
-    auto tiles = [&](int wm, int wn) {
-        return static_cast<int64_t>((n + 64 * wn - 1) / (64 * wn)) * ((b + 64 * wm - 1) / (64 * wm));
-    };
-    if (b > 128) {
-        const int64_t mt = (b + 255) / 256;
-        const int64_t t = static_cast<int64_t>((n + 127) / 128) * mt;
-        if (t >= 192) return {2, 2, 1, k, 4};
-        if (static_cast<int64_t>((n + 63) / 64) * mt >= 192) return {2, 1, 1, k, 4};
-        // fewer tiles: 256 x 128 with K split (ranges of whole 256-value
-        // blocks) until about 256 work-groups run
-        int32_t splits = static_cast<int32_t>(256 / t);
-        if (splits > k / 256) splits = k / 256;
-        if (splits <= 1) return {2, 2, 1, k, 4};
-        const int32_t kchunk = (k / 256 + splits - 1) / splits * 256;
-        return {2, 2, (k + kchunk - 1) / kchunk, kchunk, 4};
-    }
-    if (b > 64) {
-        // 128 x 128 tiles of 4 waves, with K split until about 512 work-groups run
-        const int64_t t = tiles(2, 2);
-        int32_t splits = static_cast<int32_t>(512 / t);
-        if (splits > k / 256) splits = k / 256;
-        if (splits <= 1) return {2, 2, 1, k};
-        const int32_t kchunk = (k / 256 + splits - 1) / splits * 256;
-        return {2, 2, (k + kchunk - 1) / kchunk, kchunk};
-    }
-    const int cand[3][3] = {{2, 2, 2}, {2, 1, 2}, {1, 1, 4}};
-    for (const auto& c : cand)
-        if (tiles(c[0], c[1]) >= 256 * c[2]) return {c[0], c[1], 1, k};
-    const int64_t t = tiles(1, 1);
-    int32_t splits = static_cast<int32_t>((1024 + t - 1) / t);
-    const int32_t max_splits = k / 256 > 0 ? k / 256 : 1;
-    if (splits > max_splits) splits = max_splits;
-    int32_t kchunk = (k + splits - 1) / splits;
-    kchunk = (kchunk + kMfKs - 1) / kMfKs * kMfKs;
-    splits = (k + kchunk - 1) / kchunk;
-    return {1, 1, splits, kchunk};
-}
-
-template <int TYPE, int WM, int WN, int MW = 2>
-hipError_t launch_mfma_t(const uint8_t* w, const _Float16* xhl, const float* rscale, int32_t b, int32_t k,
-                         int32_t n, float* y, const MfmaPlan& p, float* part, hipStream_t stream) {
-    constexpr int BM = 32 * WM * MW;
-    const dim3 grid((n + 64 * WN - 1) / (64 * WN), (b + BM - 1) / BM, p.splits);
-    hipLaunchKernelGGL((matbatch_mfma_kernel<TYPE, WM, WN, MW>), grid, dim3(128 * MW), 0, stream, w,
-                       row_bytes(TYPE, k), xhl, rscale, b, k, n, y, p.kchunk, part);
-    return hipGetLastError();
-}
-
-template <int TYPE>
-hipError_t launch_mfma(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, _Float16* xhl,
-                       float* rscale, float* part, hipStream_t stream, const float* up) {
-    launch_act_hilo(x, b, k, xhl, rscale, nullptr, stream, up);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const MfmaPlan p = mfma_plan(b, k, n);
-    if (p.mw == 4 && p.wn == 2) e = launch_mfma_t<TYPE, 2, 2, 4>(w, xhl, rscale, b, k, n, y, p, part, stream);
-    else if (p.mw == 4) e = launch_mfma_t<TYPE, 2, 1, 4>(w, xhl, rscale, b, k, n, y, p, part, stream);
-    else if (p.wn == 2) e = launch_mfma_t<TYPE, 2, 2>(w, xhl, rscale, b, k, n, y, p, part, stream);
-    else if (p.wm == 2) e = launch_mfma_t<TYPE, 2, 1>(w, xhl, rscale, b, k, n, y, p, part, stream);
-    else e = launch_mfma_t<TYPE, 1, 1>(w, xhl, rscale, b, k, n, y, p, part, stream);
-    if (e != hipSuccess || p.splits == 1) return e;
-    RedMats r{};
-    r.y[0] = y;
-    r.end[0] = static_cast<size_t>(b) * n;
-    r.count = 1;
-    return launch_reduce(part, p.splits, r, stream);
-}
-
-// A launch plan of matbatch_qs_stream_kernel: K ranges and the XCD order
-struct Q4kPlan {
-    int32_t splits, kchunk;
-    int32_t xmap = 0;  // token groups of the XCD-aware order (> 0), minus row groups (< 0), 0: grid order
-};
 
 // The XCD order of rg x tg work-groups with the least L2-miss traffic,
 // counting each XCD's own reads of w weight and x activation bytes: by token
@@ -1684,112 +1299,102 @@ int32_t xcd_order(int64_t rg, int64_t tg, double w, double x) {
     return tg % 8 == 0 ? static_cast<int32_t>(tg) : 0;
 }
 
-// Row groups of 256 x 64 tokens, K split in ranges of whole super-blocks
-// until about 256 work-groups run (one per CU).
-Q4kPlan q4k_stream_plan(int32_t b, int32_t k, int32_t n) {
-    Q4kPlan p{1, k};
-    const int32_t nsb = k / 256;
-    const int64_t rg = (n + 255) / 256, tg = (b + kQsTok - 1) / kQsTok, wgs = rg * tg;
-    int32_t splits = wgs >= 256 ? 1 : static_cast<int32_t>(256 / wgs);
-    splits = std::max(1, std::min(splits, nsb));
-    const int32_t csb = (nsb + splits - 1) / splits;
-    p.kchunk = csb * 256;
-    p.splits = (nsb + csb - 1) / csb;
-    p.xmap = 0;
-    if (p.splits == 1)
-        p.xmap = xcd_order(rg, tg, static_cast<double>(n) * (k / 256) * 210.0, static_cast<double>(b) * k * 2.2);
-    return p;
+// A launch plan of matbatch_qs_stream_kernel: token fragments per work-group,
+// K ranges and the XCD order (0: grid order)
+struct QsPlan {
+    int tf;
+    int32_t splits, kchunk, xmap;
+};
+
+// Row groups of 256 x 16, 32, 64 or 128 tokens and K split in ranges of whole
+// super-blocks, whichever is estimated fastest: rounds of 256 work-groups
+// (one per CU), each a fixed part and its super-blocks, and with split K the
+// reduce.  Microseconds per super-block of a work-group as measured: 64 and
+// 128 tokens on full grids (4096 x 12288, B = 2048 and 512), 16 and 32 on one
+// work-group per CU, where the latency of a super-block's loads bounds them.
+// 128-token tiles read each weight for twice the tokens, but pad short
+// batches.
+// n: the rows of all matrices of the launch.
+QsPlan qs_plan(int32_t type, int32_t b, int32_t k, int32_t n) {
+    static const double kStep[4][4] = {
+        {2.5, 3.3, 3.9, 6.4},   // Q4_K
+        {4.1, 5.0, 5.6, 9.3},   // Q6_K
+        {5.0, 6.0, 7.2, 8.8},   // Q8_0
+        {5.0, 5.8, 7.1, 8.6}};  // Q4_0
+    static const double kFixed[4] = {2.5, 3.0, 4.0, 5.0};
+    const double* step = kStep[type == kQ4_K ? 0 : type == kQ6_K ? 1 : type == kQ8_0 ? 2 : 3];
+    const int32_t nsb = (k + 255) / 256;
+    const int64_t rg = (n + kQsRows - 1) / kQsRows;
+    QsPlan best{1, 1, k, 0};
+    double least = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        const int32_t tf = 1 << i;
+        if (i < 2 && b > 32 * tf) continue;  // short tiles for short batches
+        if (i > 0 && b <= 8 * tf) break;     // none twice as wide as the batch
+        const int64_t tg = (b + 16 * tf - 1) / (16 * tf);
+        for (int32_t want = 1; want <= nsb && want <= 64; ++want) {
+            const int32_t csb = (nsb + want - 1) / want, splits = (nsb + csb - 1) / csb;
+            if (splits != want) continue;
+            const double rounds = static_cast<double>((rg * tg * splits + 255) / 256);
+            const double parts = splits > 1 ? static_cast<double>(splits) * b * n * 4.0 : 0.0;
+            const double us = rounds * (kFixed[i] + csb * step[i]) + (splits > 1 ? 3.0 + parts / 2.5e6 : 0.0);
+            if (least == 0.0 || us < least) {
+                least = us;
+                best = {tf, splits, splits > 1 ? csb * 256 : k, 0};
+            }
+        }
+    }
+    if (best.splits == 1)
+        best.xmap = xcd_order(rg, (b + 16 * best.tf - 1) / (16 * best.tf), static_cast<double>(n) * k * (210.0 / 256.0),
+                              static_cast<double>(b) * k * 2.2);
+    return best;
 }
 
-Q4kPlan q4k_plan(int32_t b, int32_t k, int32_t n) { return q4k_stream_plan(b, k, n); }
-
-// rows per row group of the streamed kernel (8 waves x 32 rows)
-constexpr int32_t kQ4kTileRows = 256;
-
-// the streamed kernel's activations: q as fp16 in xhl's first B K halves and
-// the blocks' d / s after them (the pairs' space holds both)
-float* q4k_dxs(_Float16* xhl, int32_t b, int32_t k) { return reinterpret_cast<float*>(xhl + static_cast<size_t>(b) * k); }
-
-void launch_q4k_act(const float* x, int32_t b, int32_t k, _Float16* xhl, float* rscale, _Float16* pq,
-                    hipStream_t stream, const float* up) {
-    launch_act_q(x, b, k, xhl, q4k_dxs(xhl, b, k), rscale, pq, stream, up);
-}
-
-template <int TYPE>
-hipError_t launch_qs(const MbMats& m, const _Float16* xq, const float* dxs, const _Float16* pq,
-                     const float* rscale, int32_t b, int32_t k, const Q4kPlan& p, float* part, hipStream_t stream) {
-    constexpr int BN = 256;
-    if (p.kchunk % 256 != 0) return hipErrorInvalidValue;
-    const int32_t rg = m.tile0[m.count - 1] + (m.n[m.count - 1] + BN - 1) / BN, tg = (b + kQsTok - 1) / kQsTok;
+template <int TYPE, int TF>
+hipError_t launch_qs_t(const MbMats& m, const QsBufs& q, int32_t b, int32_t k, const QsPlan& p, hipStream_t stream) {
+    const int32_t rg = m.tile0[m.count - 1] + (m.n[m.count - 1] + kQsRows - 1) / kQsRows;
+    const int32_t tg = (b + 16 * TF - 1) / (16 * TF);
+    if (p.kchunk % 256 != 0 && p.splits > 1) return hipErrorInvalidValue;
     if (p.xmap > 0 && (p.xmap != tg || tg % 8 != 0 || p.splits != 1)) return hipErrorInvalidValue;
     if (p.xmap < 0 && (-p.xmap != rg || rg % 8 != 0 || p.splits != 1)) return hipErrorInvalidValue;
     const dim3 grid = p.xmap != 0 ? dim3(rg * tg) : dim3(rg, tg, p.splits);
-    hipLaunchKernelGGL((matbatch_qs_stream_kernel<TYPE, 8>), grid, dim3(512), 0, stream, m, row_bytes(TYPE, k), xq,
-                       dxs, pq, rscale, b, k, p.kchunk, part, p.xmap);
+    hipLaunchKernelGGL((matbatch_qs_stream_kernel<TYPE, TF>), grid, dim3(512), 0, stream, m, row_bytes(TYPE, k), q.xq,
+                       q.dxs, q.pq, q.rscale, b, k, p.kchunk, q.part, p.xmap);
     return hipGetLastError();
 }
 
-#ifndef GNCX_Q6K_STREAM
-#define GNCX_Q6K_STREAM 1
-#endif
-// Q6_K through matbatch_qs_stream_kernel (plan as q4k_stream_plan): the
-// activations as q, d / s and row scales, the product, with split K the
-// reduce
-hipError_t launch_q6ks(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, _Float16* xhl,
-                       float* rscale, float* part, hipStream_t stream, const float* up) {
-    const Q4kPlan p = q4k_stream_plan(b, k, n);
-    launch_act_q(x, b, k, xhl, q4k_dxs(xhl, b, k), rscale, nullptr, stream, up);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    MbMats m{};
-    m.w[0] = w;
-    m.y[0] = y;
-    m.n[0] = n;
-    m.ntot = n;
-    m.count = 1;
-    e = launch_qs<kQ6_K>(m, xhl, q4k_dxs(xhl, b, k), nullptr, rscale, b, k, p, part, stream);
-    if (e != hipSuccess || p.splits == 1) return e;
-    RedMats r{};
-    r.y[0] = y;
-    r.end[0] = static_cast<size_t>(b) * n;
-    r.count = 1;
-    return launch_reduce(part, p.splits, r, stream);
+template <int TYPE>
+hipError_t launch_qs_tf(const MbMats& m, const QsBufs& q, int32_t b, int32_t k, const QsPlan& p, hipStream_t stream) {
+    return p.tf == 1   ? launch_qs_t<TYPE, 1>(m, q, b, k, p, stream)
+           : p.tf == 2 ? launch_qs_t<TYPE, 2>(m, q, b, k, p, stream)
+           : p.tf == 4 ? launch_qs_t<TYPE, 4>(m, q, b, k, p, stream)
+                       : launch_qs_t<TYPE, 8>(m, q, b, k, p, stream);
 }
 
-// The product of plan p over the matrices of m (w, y, n and count set), then
-// with split K the reduce of the partials into each y
-hipError_t launch_q4k_mats(MbMats& m, _Float16* xhl, const _Float16* pq, const float* rscale, int32_t b,
-                           int32_t k, const Q4kPlan& p, float* part, hipStream_t stream) {
-    const int32_t bn = kQ4kTileRows;
+// The product of plan p over the matrices of m (w, y, n and count set) from
+// the quantised activations in q, then with split K the reduce of the
+// partials into each y
+hipError_t launch_qs(int32_t type, MbMats& m, const QsBufs& q, int32_t b, int32_t k, const QsPlan& p,
+                     hipStream_t stream) {
     int32_t t = 0, rows = 0;
     RedMats r{};
     for (int32_t i = 0; i < m.count; ++i) {
         m.tile0[i] = t;
         m.npre[i] = rows;
-        t += (m.n[i] + bn - 1) / bn;
+        t += (m.n[i] + kQsRows - 1) / kQsRows;
         rows += m.n[i];
         r.y[i] = m.y[i];
         r.end[i] = static_cast<size_t>(b) * rows;
     }
     m.ntot = rows;
     r.count = m.count;
-    const hipError_t e = launch_qs<kQ4_K>(m, xhl, q4k_dxs(xhl, b, k), pq, rscale, b, k, p, part, stream);
+    hipError_t e = hipErrorInvalidValue;
+    if (type == kQ4_K) e = launch_qs_tf<kQ4_K>(m, q, b, k, p, stream);
+    else if (type == kQ6_K) e = launch_qs_tf<kQ6_K>(m, q, b, k, p, stream);
+    else if (type == kQ8_0) e = launch_qs_tf<kQ8_0>(m, q, b, k, p, stream);
+    else if (type == kQ4_0) e = launch_qs_tf<kQ4_0>(m, q, b, k, p, stream);
     if (e != hipSuccess || p.splits == 1) return e;
-    return launch_reduce(part, p.splits, r, stream);
-}
-
-hipError_t launch_q4k(const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n, float* y, _Float16* xhl,
-                      _Float16* pq, float* rscale, float* part, hipStream_t stream, const float* up) {
-    const Q4kPlan p = q4k_plan(b, k, n);
-    launch_q4k_act(x, b, k, xhl, rscale, pq, stream, up);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    MbMats m{};
-    m.w[0] = w;
-    m.y[0] = y;
-    m.n[0] = n;
-    m.count = 1;
-    return launch_q4k_mats(m, xhl, pq, rscale, b, k, p, part, stream);
+    return launch_reduce(q.part, p.splits, r, stream);
 }
 
 // BF16: 256 rows per row group and 16, 32 or 64 tokens, K split in ranges of
@@ -1853,18 +1458,32 @@ hipError_t launch_bf16(const uint8_t* w, const float* x, int32_t b, int32_t k, i
 
 }  // namespace
 
-// fp16 pairs of the quantised activations [B x K x 2] (or, for the
-// streamed Q4_K / Q6_K kernel, q [B x K] and the blocks' d / s [B x K / 32]),
-// their row scales [B], then the split-K partials [splits x B x N]
-static size_t xh_bytes(int32_t b, int32_t k) {
-    return (static_cast<size_t>(b) * k * 2 * sizeof(_Float16) + 255) & ~static_cast<size_t>(255);
+static size_t pad256(size_t v) { return (v + 255) & ~size_t{255}; }
+// q [B x K] as fp16 and the blocks' d / s [B x K / 32]
+static size_t xq_bytes(int32_t b, int32_t k) {
+    return pad256(static_cast<size_t>(b) * k * sizeof(_Float16) + static_cast<size_t>(b) * (k / 32) * sizeof(float));
 }
-static size_t rscale_bytes(int32_t b) { return (static_cast<size_t>(b) * sizeof(float) + 255) & ~static_cast<size_t>(255); }
+static size_t rscale_bytes(int32_t b) { return pad256(static_cast<size_t>(b) * sizeof(float)); }
 
 // Q4_K: the activation sums of each 32-block as fp16 pairs [B x K/256 x 16]
 static size_t pq_bytes(int32_t type, int32_t b, int32_t k) {
-    return type == kQ4_K ? (static_cast<size_t>(b) * (k / 256) * 16 * sizeof(_Float16) + 255) & ~static_cast<size_t>(255)
-                         : 0;
+    return type == kQ4_K ? pad256(static_cast<size_t>(b) * (k / 256) * 16 * sizeof(_Float16)) : 0;
+}
+
+static size_t qs_bytes(int32_t type, int32_t b, int32_t k, int64_t n, int32_t splits) {
+    const size_t parts = splits > 1 ? static_cast<size_t>(splits) * b * n * sizeof(float) : 0;
+    return xq_bytes(b, k) + pq_bytes(type, b, k) + rscale_bytes(b) + parts + 256;
+}
+
+static QsBufs qs_bufs(void* workspace, int32_t type, int32_t b, int32_t k) {
+    char* ws = static_cast<char*>(workspace);
+    QsBufs q;
+    q.xq = reinterpret_cast<_Float16*>(ws);
+    q.dxs = reinterpret_cast<float*>(q.xq + static_cast<size_t>(b) * k);
+    q.pq = type == kQ4_K ? reinterpret_cast<_Float16*>(ws + xq_bytes(b, k)) : nullptr;
+    q.rscale = reinterpret_cast<float*>(ws + xq_bytes(b, k) + pq_bytes(type, b, k));
+    q.part = reinterpret_cast<float*>(ws + xq_bytes(b, k) + pq_bytes(type, b, k) + rscale_bytes(b));
+    return q;
 }
 
 size_t matbatch_workspace_bytes(int32_t type, int32_t b, int32_t k, int32_t n) {
@@ -1872,11 +1491,7 @@ size_t matbatch_workspace_bytes(int32_t type, int32_t b, int32_t k, int32_t n) {
         const int32_t splits = bf16_small(b, k, n) ? 1 : bf16_plan(b, k, n).splits;
         return (splits > 1 ? static_cast<size_t>(splits) * b * n * sizeof(float) : 0) + 256;
     }
-    const int32_t splits = type == kQ4_K                     ? q4k_plan(b, k, n).splits
-                           : type == kQ6_K && GNCX_Q6K_STREAM ? q4k_stream_plan(b, k, n).splits
-                                                              : mfma_plan(b, k, n).splits;
-    const size_t parts = splits > 1 ? static_cast<size_t>(splits) * b * n * sizeof(float) : 0;
-    return xh_bytes(b, k) + pq_bytes(type, b, k) + rscale_bytes(b) + parts + 256;
+    return qs_bytes(type, b, k, n, qs_plan(type, b, k, n).splits);
 }
 
 hipError_t launch_matbatch(int32_t type, const uint8_t* w, const float* x, int32_t b, int32_t k, int32_t n,
@@ -1893,24 +1508,21 @@ hipError_t launch_matbatch(int32_t type, const uint8_t* w, const float* x, int32
     } else if ((wa & 3u) != 0) {
         return hipErrorInvalidValue;
     }
-    char* ws = static_cast<char*>(workspace);
-    _Float16* xhl = reinterpret_cast<_Float16*>(ws);
-    _Float16* pq = reinterpret_cast<_Float16*>(ws + xh_bytes(b, k));
-    float* rscale = reinterpret_cast<float*>(ws + xh_bytes(b, k) + pq_bytes(type, b, k));
-    float* part = reinterpret_cast<float*>(ws + xh_bytes(b, k) + pq_bytes(type, b, k) + rscale_bytes(b));
-    if ((reinterpret_cast<uintptr_t>(xhl) & 255u) != 0) return hipErrorInvalidValue;
-    switch (type) {
-    case kQ4_0: return launch_mfma<kQ4_0>(w, x, b, k, n, y, xhl, rscale, part, stream, up);
-    case kQ8_0: return launch_mfma<kQ8_0>(w, x, b, k, n, y, xhl, rscale, part, stream, up);
-    case kQ4_K: return launch_q4k(w, x, b, k, n, y, xhl, pq, rscale, part, stream, up);
-    case kQ6_K:
-        return GNCX_Q6K_STREAM ? launch_q6ks(w, x, b, k, n, y, xhl, rscale, part, stream, up)
-                               : launch_mfma<kQ6_K>(w, x, b, k, n, y, xhl, rscale, part, stream, up);
-    case kBF16: return up ? hipErrorNotSupported : launch_bf16(w, x, b, k, n, y, static_cast<float*>(workspace), stream);
-    default: return hipErrorInvalidValue;
-    }
+    if (type == kBF16)
+        return up ? hipErrorNotSupported : launch_bf16(w, x, b, k, n, y, static_cast<float*>(workspace), stream);
+    if (type != kQ4_0 && type != kQ8_0 && type != kQ4_K && type != kQ6_K) return hipErrorInvalidValue;
+    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return hipErrorInvalidValue;
+    const QsBufs q = qs_bufs(workspace, type, b, k);
+    launch_act_q(x, b, k, q, stream, up);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    MbMats m{};
+    m.w[0] = w;
+    m.y[0] = y;
+    m.n[0] = n;
+    m.count = 1;
+    return launch_qs(type, m, q, b, k, qs_plan(type, b, k, n), stream);
 }
-
 
 namespace {
 
@@ -1918,15 +1530,14 @@ namespace {
 // split K one reduce over all of them): when every matrix is whole x-tiles of
 // the plan for the summed rows (false otherwise, and the matrices go one call
 // each).
-bool multi_fused(int32_t type, int32_t count, const int32_t* ns, int32_t b, int32_t k, Q4kPlan& p, int64_t& total) {
+bool multi_fused(int32_t type, int32_t count, const int32_t* ns, int32_t b, int32_t k, QsPlan& p, int64_t& total) {
     if (type != kQ4_K || count < 2 || count > kMaxMbMats || b <= 0 || k <= 0 || (k % 256) != 0) return false;
     total = 0;
     for (int32_t i = 0; i < count; ++i) total += ns[i];
     if (total > INT32_MAX) return false;
-    p = q4k_plan(b, k, static_cast<int32_t>(total));
-    const int32_t bn = kQ4kTileRows;
+    p = qs_plan(type, b, k, static_cast<int32_t>(total));
     for (int32_t i = 0; i < count; ++i)
-        if (ns[i] % bn != 0) return false;
+        if (ns[i] % kQsRows != 0) return false;
     return true;
 }
 
@@ -1935,11 +1546,10 @@ bool multi_fused(int32_t type, int32_t count, const int32_t* ns, int32_t b, int3
 size_t matbatch_multi_workspace_bytes(int32_t type, int32_t count, const int32_t* ns, int32_t b, int32_t k) {
     size_t need = 256;
     for (int32_t i = 0; i < count; ++i) need = std::max(need, matbatch_workspace_bytes(type, b, k, ns[i]));
-    Q4kPlan p;
+    QsPlan p;
     int64_t total;
     if (multi_fused(type, count, ns, b, k, p, total)) {
-        const size_t parts = p.splits > 1 ? static_cast<size_t>(p.splits) * b * total * sizeof(float) : 0;
-        need = std::max(need, xh_bytes(b, k) + pq_bytes(type, b, k) + rscale_bytes(b) + parts + 256);
+        need = std::max(need, qs_bytes(type, b, k, total, p.splits));
     }
     return need;
 }
@@ -1951,7 +1561,7 @@ hipError_t launch_matbatch_multi(int32_t type, int32_t count, const uint8_t* con
     for (int32_t i = 0; i < count; ++i)
         if (ns[i] <= 0 || !ws[i] || !ys[i]) return hipErrorInvalidValue;
     if (workspace_bytes < matbatch_multi_workspace_bytes(type, count, ns, b, k)) return hipErrorInvalidValue;
-    Q4kPlan p;
+    QsPlan p;
     int64_t total;
     if (!multi_fused(type, count, ns, b, k, p, total)) {
         for (int32_t i = 0; i < count; ++i) {
@@ -1965,13 +1575,9 @@ hipError_t launch_matbatch_multi(int32_t type, int32_t count, const uint8_t* con
     if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0 || (row_bytes(kQ4_K, k) & 15u) != 0) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
         if ((reinterpret_cast<uintptr_t>(ws[i]) & 15u) != 0) return hipErrorInvalidValue;
-    char* wsp = static_cast<char*>(workspace);
-    _Float16* xhl = reinterpret_cast<_Float16*>(wsp);
-    _Float16* pq = reinterpret_cast<_Float16*>(wsp + xh_bytes(b, k));
-    float* rscale = reinterpret_cast<float*>(wsp + xh_bytes(b, k) + pq_bytes(kQ4_K, b, k));
-    float* part = reinterpret_cast<float*>(wsp + xh_bytes(b, k) + pq_bytes(kQ4_K, b, k) + rscale_bytes(b));
-    if ((reinterpret_cast<uintptr_t>(xhl) & 255u) != 0) return hipErrorInvalidValue;
-    launch_q4k_act(x, b, k, xhl, rscale, pq, stream, nullptr);
+    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return hipErrorInvalidValue;
+    const QsBufs q = qs_bufs(workspace, type, b, k);
+    launch_act_q(x, b, k, q, stream, nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     MbMats m{};
@@ -1981,7 +1587,7 @@ hipError_t launch_matbatch_multi(int32_t type, int32_t count, const uint8_t* con
         m.n[i] = ns[i];
     }
     m.count = count;
-    return launch_q4k_mats(m, xhl, pq, rscale, b, k, p, part, stream);
+    return launch_qs(type, m, q, b, k, p, stream);
 }
 
 hipError_t launch_matbatch_multi_norm(int32_t type, int32_t count, const uint8_t* const* ws, const int32_t* ns,
@@ -1991,20 +1597,16 @@ hipError_t launch_matbatch_multi_norm(int32_t type, int32_t count, const uint8_t
     if (count <= 0 || count > kMaxMbMats || !ws || !ns || !ys || !h || !gamma) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
         if (ns[i] <= 0 || !ws[i] || !ys[i]) return hipErrorInvalidValue;
-    Q4kPlan p;
+    QsPlan p;
     int64_t total;
     if (!multi_fused(type, count, ns, b, k, p, total) || !norm_act_fits(h, r, gamma, k)) return hipErrorNotSupported;
     if (workspace_bytes < matbatch_multi_workspace_bytes(type, count, ns, b, k)) return hipErrorInvalidValue;
     if (k > (1 << 20) || b > 65535 || (row_bytes(kQ4_K, k) & 15u) != 0) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
         if ((reinterpret_cast<uintptr_t>(ws[i]) & 15u) != 0) return hipErrorInvalidValue;
-    char* wsp = static_cast<char*>(workspace);
-    _Float16* xhl = reinterpret_cast<_Float16*>(wsp);
-    _Float16* pq = reinterpret_cast<_Float16*>(wsp + xh_bytes(b, k));
-    float* rscale = reinterpret_cast<float*>(wsp + xh_bytes(b, k) + pq_bytes(kQ4_K, b, k));
-    float* part = reinterpret_cast<float*>(wsp + xh_bytes(b, k) + pq_bytes(kQ4_K, b, k) + rscale_bytes(b));
-    if ((reinterpret_cast<uintptr_t>(xhl) & 255u) != 0) return hipErrorInvalidValue;
-    launch_norm_act_q(h, r, gamma, eps, b, k, xhl, q4k_dxs(xhl, b, k), rscale, pq, stream);
+    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return hipErrorInvalidValue;
+    const QsBufs q = qs_bufs(workspace, type, b, k);
+    launch_norm_act_q(h, r, gamma, eps, b, k, q, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     MbMats m{};
@@ -2014,7 +1616,7 @@ hipError_t launch_matbatch_multi_norm(int32_t type, int32_t count, const uint8_t
         m.n[i] = ns[i];
     }
     m.count = count;
-    return launch_q4k_mats(m, xhl, pq, rscale, b, k, p, part, stream);
+    return launch_qs(type, m, q, b, k, p, stream);
 }
 
 }  // namespace gncx

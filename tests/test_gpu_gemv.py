@@ -4,9 +4,9 @@ Bars: Q8 activation blocks and block dequantisation bit-exact with the
 oracle; matvec / matbatch / lm_head within 1e-3 relative L2 of the oracle's
 fp32 results on the same seeded inputs.  matvec keeps the integer block dots
 (only fp32 accumulation order differs: ~1e-7).  matbatch of quantised weights
-runs on fp16 matrix cores with both operands as fp16 (hi, lo) pairs, three
-products per K slice, which is held to 1e-5 (measured ~2e-7): a kernel that
-dropped a lo term, or rounded either operand to one fp16, lands near 3e-4."""
+runs on fp16 matrix cores with exact integer operands and block dots, held to
+1e-5 (measured ~1e-7): a kernel that rounded either operand to one fp16 lands
+near 3e-4."""
 from __future__ import annotations
 
 import ctypes as C
@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 Q4_0, Q8_0, Q4_K, Q6_K, BF16 = 2, 8, 12, 14, 30
 TOL = 1e-3  # relative L2, fp32 outputs
-TOL_MATBATCH = 1e-5  # the fp16-pair products of matbatch (quantised types)
+TOL_MATBATCH = 1e-5  # matbatch of the quantised types
 
 
 def test_act_quant_bitexact(lib, oracle):
@@ -326,6 +326,32 @@ def test_matbatch_bf16_infinite_and_nan(lib):
     assert np.array_equal(np.sign(y[big]), np.sign(want[big]))
     inf = np.isinf(want)
     assert np.array_equal(y[inf], want[inf].astype(np.float32))
+
+
+# The streamed kernel's token tiles (16, 32, 64, 128) at their edges, Q8_0 and
+# Q4_0 rows that end inside a 256-value super-block (one block, and one more
+# than whole ones), K ranges that do, row groups of fewer than 256 rows and
+# rows at odd 2-byte addresses.
+STREAM_CASES = [(Q8_0, 32, 5, 1), (Q4_0, 288, 601, 17), (Q6_K, 512, 33, 16), (Q8_0, 2080, 4101, 700),
+                (Q4_0, 4128, 301, 129), (Q4_K, 512, 7000, 1000), (Q6_K, 768, 5000, 1100), (Q4_0, 32, 20001, 400),
+                (Q8_0, 14368, 257, 65), (Q4_0, 14368, 300, 33), (Q8_0, 4096, 255, 128), (Q4_K, 768, 257, 128)]
+
+
+@pytest.mark.parametrize("t,k,n,b", STREAM_CASES)
+def test_matbatch_stream_tiles(lib, oracle, t, k, n, b):
+    w = synth.make_weights(t, n, k, seed=3100 + t + k + n)
+    x = synth.make_activations(b, k, seed=4100 + t + k + b).reshape(b, k).copy()
+    x[:, :32] = 0.0  # a zero block (scale 0) in every row
+    y = np.full((b, n), np.nan, np.float32)
+    lib.gncx_xfold_universal_matbatch(ptr(w), 0, t, ptr(x), b, k, n, ptr(y), None)
+    gncx.check(lib)
+    want = oracle.matbatch(t, w, x, b, k, n)
+    if not np.any(want):
+        assert not np.any(y)
+        return
+    # exact block dots: a chain of at most 8 + K / 256 + 64 fp32 roundings of
+    # 2^-24, random in sign (measured 0.7e-7 to 1.3e-7)
+    assert rel_l2(y, want) < 5e-7
 
 
 # Q6_K scales beyond +-64 (real quantisers use the whole int8 range): then
