@@ -409,6 +409,31 @@ def test_attention_prefill_equals_fused_steps(lib, H, KV, hd, pos0, B, sw):
     assert max(errs) < 1e-5
 
 
+# the batched prologue takes 16 heads per work-group: fewer, whole and partial
+# groups, q and KV heads in one group, without weight, without rotation, and
+# weights at a 4-byte aligned offset
+@pytest.mark.parametrize("H,KV,weight,base,off", [(2, 1, 1, 1e6, 0), (16, 16, 0, 1e6, 0), (32, 8, 1, 0.0, 4),
+                                                  (12, 3, 1, 1e4, 4), (28, 7, 0, 0.0, 0)])
+def test_attention_prefill_prologue_bitexact(lib, H, KV, weight, base, off):
+    hd, pos0, B, scale, eps = 128, 3, 9, 1 / np.sqrt(128), 1e-6
+    kc, vc, q, k, v, norms = _prefill_inputs(H, KV, hd, pos0, B, H * 100 + KV)
+    norms = np.concatenate([np.zeros(off // 4, np.float32), norms])
+    q1, k1, kc1, vc1 = q.copy(), k.copy(), kc.copy(), vc.copy()
+    out = np.zeros((B, H * hd), np.float32)
+    for t in range(B):
+        lib.gncx_hip_attention_step_fused(ptr(q1[t]), ptr(k1[t]), ptr(v[t]), ptr(kc1), ptr(vc1), pos0 + t, H, KV, hd,
+                                          scale, 0, 1, ptr(norms), off, off + hd * 4, weight, eps, 0, 0, base,
+                                          ptr(out[t]))
+    gncx.check(lib)
+    lib.gncx_hip_kv_forget(None)
+    lib.gncx_hip_attention_prefill(ptr(q), ptr(k), ptr(v), ptr(kc), ptr(vc), pos0, B, H, KV, hd, scale, 0, ptr(norms),
+                                   off, off + hd * 4, weight, eps, 0, 0, base, ptr(out))
+    gncx.check(lib)
+    lib.gncx_hip_kv_forget(None)
+    assert np.array_equal(q1, q) and np.array_equal(k1, k)
+    assert np.array_equal(kc1, kc) and np.array_equal(vc1, vc)
+
+
 @pytest.mark.parametrize("pos0,B,sw", [(10, 64, 0), (300, 200, 0), (0, 600, 200)])
 def test_attention_prefill_device_buffers(lib, oracle, pos0, B, sw):
     """Device-resident buffers (used in place), against the oracle's
