@@ -210,6 +210,10 @@ constexpr int kNormStride = 64 * kNormWaves;
 
 enum BandSched { kSchedOne = 1, kSchedTwo = 2 };
 
+// the ggml type behind a slot type
+constexpr int32_t ggml_type_of(int type) { return type == kBF16Wide ? kBF16 : type; }
+constexpr bool is_bf16(int type) { return ggml_type_of(type) == kBF16; }
+
 // x tasks (4 values) per quantising thread with loads in flight together,
 // and the least number of quantising waves
 template <int SCHED>
@@ -287,12 +291,12 @@ __global__ __launch_bounds__(THREADS) void gemv_band_kernel(BandMats mats, uint3
                                                                  const float* __restrict x, int32_t k,
                                                                  int32_t n, int32_t nwk, int32_t nwr, int32_t nqw,
                                                                  BandExtra ex) {
-    static_assert(EXT == kExtNone || (SCHED == kSchedOne && THREADS == 1024 && TYPE != kBF16),
+    static_assert(EXT == kExtNone || (SCHED == kSchedOne && THREADS == 1024 && !is_bf16(TYPE)),
                   "fused prologue / epilogue: ONE schedule, 1024 threads, quantised weights");
     using S = Slot<TYPE>;
     using Frag = typename S::Frag;
     using Act = typename S::Act;
-    constexpr bool kQuant = TYPE != kBF16;
+    constexpr bool kQuant = !is_bf16(TYPE);
     constexpr int kU = BandQuant<SCHED>::kU;
     extern __shared__ __align__(16) uint8_t lds[];
     int32_t* ctl = reinterpret_cast<int32_t*>(lds);
@@ -374,7 +378,9 @@ __global__ __launch_bounds__(THREADS) void gemv_band_kernel(BandMats mats, uint3
                 __builtin_amdgcn_s_sleep(1);
             asm volatile("" ::: "memory");
         }
-        if (has_slot) slot_act<TYPE>(a, s, q, meta, x);
+        if (!has_slot) return;
+        if constexpr (TYPE == kBF16Wide) S::load_act_x(a, s, x, k);
+        else slot_act<TYPE>(a, s, q, meta, x);
     };
 
     Frag fa, fb;
@@ -593,9 +599,9 @@ template <int TYPE, int THREADS, int SCHED>
 bool try_band_sched(const BandMats& m, const float* x, int32_t k, int32_t n, hipStream_t stream) {
     int32_t groups, nwk, nwr, nqw;
     size_t lds;
-    if (!band_plan(Slot<TYPE>::slots(k), k, n, TYPE != kBF16, THREADS / 64, SCHED, groups, nwk, nwr, nqw, lds))
+    if (!band_plan(Slot<TYPE>::slots(k), k, n, !is_bf16(TYPE), THREADS / 64, SCHED, groups, nwk, nwr, nqw, lds))
         return false;
-    const uint32_t rb = static_cast<uint32_t>(row_bytes(TYPE, k));
+    const uint32_t rb = static_cast<uint32_t>(row_bytes(ggml_type_of(TYPE), k));
     if (m.count > 1)
         hipLaunchKernelGGL((gemv_band_kernel<TYPE, THREADS, SCHED, true>), dim3(groups), dim3(THREADS), lds, stream, m,
                            rb, x, k, n, nwk, nwr, nqw, BandExtra{});
@@ -647,12 +653,14 @@ bool try_band_ext_type(int32_t type, const BandMats& m, const float* x, int32_t 
 // ONE for 16-wave groups with at least kOneMinRowWaves row-waves, and for
 // Q4_K / Q8_0 rows split into three or more K-slices (Q4_K 12288 x 4096:
 // 8.2 vs 8.8 us under TWO; Q8_0 14336 x 4096: 14.3 vs 15.5 us); TWO otherwise
+// (BF16: TWO; the wide slots read zeros past the row only through its buffers)
 template <int TYPE, int THREADS>
 bool try_band(const BandMats& m, const float* x, int32_t k, int32_t n, hipStream_t stream) {
     const int32_t nwk = (Slot<TYPE>::slots(k) + 63) / 64;
     const bool one = nwk >= 1 && ((THREADS / 64) / nwk >= kOneMinRowWaves ||
                                   (nwk >= 3 && (TYPE == kQ4_K || TYPE == kQ8_0)));
-    if (THREADS == 1024 && one && try_band_sched<TYPE, THREADS, kSchedOne>(m, x, k, n, stream)) return true;
+    if constexpr (THREADS == 1024 && !is_bf16(TYPE))
+        if (one && try_band_sched<TYPE, THREADS, kSchedOne>(m, x, k, n, stream)) return true;
     return try_band_sched<TYPE, THREADS, kSchedTwo>(m, x, k, n, stream);
 }
 
@@ -660,10 +668,16 @@ bool try_band(const BandMats& m, const float* x, int32_t k, int32_t n, hipStream
 template <int TYPE>
 hipError_t launch_band(const BandMats& m, const float* x, int32_t k, int32_t n, hipStream_t stream, bool& used) {
     const int32_t groups = n < kBandGroups ? n : kBandGroups;
-    const size_t per_group = row_bytes(TYPE, k) * static_cast<size_t>(n) / static_cast<size_t>(groups);
+    const size_t per_group = row_bytes(ggml_type_of(TYPE), k) * static_cast<size_t>(n) / static_cast<size_t>(groups);
     // Long-K Q6_K (three or more K-slices) also streams best with 16 waves:
     // 14336 x 4096 12.5-12.7 us against 13.3-13.7 with 8, 12288 x 4096 11.1
-    // against 12.0-12.3 (the same boxes, back-to-back calls on 16 copies)
+    // against 12.0-12.3 (the same boxes, back-to-back calls on 16 copies).
+    // BF16 takes 16 waves at every size: with 8 (16 KB of a row in flight per
+    // CU) 4096 x 14336 took 31.3 us against 20.1, 4096 x 100000 198 against 123
+    if constexpr (is_bf16(TYPE)) {
+        used = try_band<TYPE, kBandThreads>(m, x, k, n, stream);
+        return used ? hipGetLastError() : hipSuccess;
+    }
     used = (per_group > kBandStreamBytes && try_band<TYPE, kBandThreadsStream>(m, x, k, n, stream)) ||
            try_band<TYPE, kBandThreads>(m, x, k, n, stream);
     return used ? hipGetLastError() : hipSuccess;
@@ -676,7 +690,16 @@ hipError_t launch_band_type(int32_t type, const BandMats& m, const float* x, int
     case kQ8_0: return launch_band<kQ8_0>(m, x, k, n, stream, used);
     case kQ4_K: return launch_band<kQ4_K>(m, x, k, n, stream, used);
     case kQ6_K: return launch_band<kQ6_K>(m, x, k, n, stream, used);
-    case kBF16: return launch_band<kBF16>(m, x, k, n, stream, used);
+    case kBF16: {
+        // 16-byte slots where a row's K-slices fill the 16 waves twice (K from
+        // 3585 to 4096), else two pieces per lane.  Narrow / wide: 4096 x 4096
+        // 7.55 / 7.75 us, 4096 x 100000 123 / 131; 1024 x 50000 22.6 / 18.0,
+        // 5000 x 7000 15.2 / 12.7, 8192 x 8192 24.3 / 23.4; past K = 8192 the
+        // narrow slots do not fit 16 waves (gemv_kernel): 14336 x 4096 31.4 /
+        // 21.3, 16384 x 5000 53.6 / 29.2
+        const bool narrow = (Slot<kBF16>::slots(k) + 63) / 64 == 8;
+        return narrow ? launch_band<kBF16>(m, x, k, n, stream, used) : launch_band<kBF16Wide>(m, x, k, n, stream, used);
+    }
     default: used = false; return hipErrorInvalidValue;
     }
 }

@@ -409,6 +409,46 @@ struct Slot<kBF16> {
     }
 };
 
+// BF16 rows in slots of two 8-weight pieces, 64 pieces apart, so that both of
+// a wave's loads are contiguous: slot s is pieces p = 128 (s / 64) + s % 64
+// and p + 64 (a row's last slice may lack the second; its weights must read
+// as zeros past the row).  For the band GEMV: twice the bytes in flight per
+// wave, and rows up to 16384 values within 16 waves.
+constexpr int kBF16Wide = 1000 + kBF16;
+template <>
+struct Slot<kBF16Wide> {
+    struct Frag {
+        u32x4 w[2];
+    };
+    struct Act {
+        float4 v[4];
+    };
+    static constexpr int32_t slots(int32_t k) {
+        const int32_t pieces = k / 8, rest = pieces % 128;
+        return pieces / 128 * 64 + (rest < 64 ? rest : 64);
+    }
+    __device__ static __forceinline__ int piece(int s) { return 128 * (s >> 6) + (s & 63); }
+    template <class Row>
+    __device__ static __forceinline__ void load(Frag& f, const Row& row, int s) {
+        const uint32_t o = static_cast<uint32_t>(piece(s)) * 16u;
+        f.w[0] = row.ld16(o);
+        f.w[1] = row.ld16(o + 1024u);
+    }
+    __device__ static __forceinline__ void load_act_x(Act& a, int s, const float* __restrict x, int32_t k) {
+        const int e = 8 * piece(s);
+        a.v[0] = *reinterpret_cast<const float4*>(x + e);
+        a.v[1] = *reinterpret_cast<const float4*>(x + e + 4);
+        const bool two = e + 512 < k;
+        a.v[2] = two ? *reinterpret_cast<const float4*>(x + e + 512) : make_float4(0.f, 0.f, 0.f, 0.f);
+        a.v[3] = two ? *reinterpret_cast<const float4*>(x + e + 516) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    __device__ static __forceinline__ float dot(const Frag& f, const Act& x, int s) {
+#pragma clang fp contract(off)
+        const Slot<kBF16>::Act lo{x.v[0], x.v[1]}, hi{x.v[2], x.v[3]};
+        return Slot<kBF16>::dot({f.w[0]}, lo, s) + Slot<kBF16>::dot({f.w[1]}, hi, s);
+    }
+};
+
 // activations of slot s from the quantised vector (LDS or global) or, for
 // BF16, from the fp32 vector
 template <int TYPE>

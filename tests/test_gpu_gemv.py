@@ -91,6 +91,25 @@ def test_matvec_parity(lib, oracle, t, k, n):
     assert err < TOL
 
 
+# BF16 rows in slots of two 8-weight pieces (every K but 3585 to 4096): one
+# piece, 64 pieces, one more, a last slice with and without second pieces, the
+# longest row that fits 16 waves and one past it, and rows of the narrow slots
+@pytest.mark.parametrize("k,n", [(8, 5), (512, 300), (520, 257), (1024, 1000), (1544, 33), (2040, 700), (3584, 65),
+                                 (3592, 300), (4096, 1030), (4104, 300), (16384, 70), (16392, 40)])
+def test_matvec_bf16_slots(lib, k, n):
+    w = synth.make_weights(BF16, n, k, seed=1100 + k + n)
+    x = synth.make_activations(1, k, seed=2100 + k + n)
+    y = np.full(n, np.nan, np.float32)
+    lib.gncx_xfold_universal_matvec(ptr(w), 0, BF16, ptr(x), None, k, n, ptr(y), None)
+    gncx.check(lib)
+    # against 64 bits (the oracle's own chain of 16384 fp32 adds is 1e-6 off):
+    # 16 products and adds per lane, 6 lane steps and up to 16 slices, each
+    # rounding at most 2^-24 of its partial sum, random in sign: sqrt(38) 2^-24
+    # = 3.7e-7 (measured about 1e-7)
+    wf = (w.view(np.uint16).astype(np.uint32) << 16).view(np.float32).reshape(n, k).astype(np.float64)
+    assert rel_l2(y, wf @ x.astype(np.float64)) < 5e-7
+
+
 def test_matvec_lm_head_shape(lib, oracle):
     """Q6_K 4096 -> 128256 (the Llama-3 lm_head GEMV)."""
     t, k, n = Q6_K, 4096, 128256
