@@ -378,9 +378,11 @@ __global__ __launch_bounds__(THREADS) void gemv_band_kernel(BandMats mats, uint3
                 __builtin_amdgcn_s_sleep(1);
             asm volatile("" ::: "memory");
         }
-        if (!has_slot) return;
-        if constexpr (TYPE == kBF16Wide) S::load_act_x(a, s, x, k);
-        else slot_act<TYPE>(a, s, q, meta, x);
+        if constexpr (TYPE == kBF16Wide) {
+            if (has_slot) S::load_act_x(a, s, x, k);
+        } else {
+            if (has_slot) slot_act<TYPE>(a, s, q, meta, x);
+        }
     };
 
     Frag fa, fb;

@@ -6,8 +6,8 @@ The oracle side restates GNCXStreamer:forward_token for the Qwen3 branch
 NEOX RoPE, attention with a KV write at pos, output projection and residual,
 RMSNorm, gate/up, SwiGLU, down and residual, then the final norm and the tied
 Q6_K lm_head.  Bar: logits within 1e-3 relative L2 at every step, for decode
-steps and for prefill (whose projections run through matbatch with fp16-pair
-operands, within ~2e-7 of the integer block dots), teacher-forced on both
+steps and for prefill (whose projections run through matbatch with exact
+integer block dots, within ~1e-7), teacher-forced on both
 sides."""
 from __future__ import annotations
 

@@ -254,7 +254,7 @@ def test_matvec_device_pointers(lib, oracle):
     assert rel_l2(yh, oracle.matvec(Q4_K, w, x, k, n)) < TOL
 
 
-# quantised types run on the fp16 matrix cores with fp16-pair operands; cases
+# quantised types run on the fp16 matrix cores with exact integer operands; cases
 # cover every tile size the launcher picks, split K, ragged B and N, and K with
 # an odd number of 32-wide steps (k % 64 == 32)
 MATBATCH_CASES = [
@@ -353,6 +353,9 @@ def test_matbatch_bf16_infinite_and_nan(lib):
 # rows at odd 2-byte addresses.
 STREAM_CASES = [(Q8_0, 32, 5, 1), (Q4_0, 288, 601, 17), (Q6_K, 512, 33, 16), (Q8_0, 2080, 4101, 700),
                 (Q4_0, 4128, 301, 129), (Q4_K, 512, 7000, 1000), (Q6_K, 768, 5000, 1100), (Q4_0, 32, 20001, 400),
+                # Q6_K matrices of an odd number of 2-byte halves of a dword (odd rows and
+                # super-blocks): the last row's scale ends in a partial dword
+                (Q6_K, 768, 33, 9), (Q6_K, 1792, 2151, 337), (Q6_K, 1280, 275, 6),
                 (Q8_0, 14368, 257, 65), (Q4_0, 14368, 300, 33), (Q8_0, 4096, 255, 128), (Q4_K, 768, 257, 128)]
 
 
