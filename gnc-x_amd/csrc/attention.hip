@@ -1338,7 +1338,7 @@ constexpr size_t kPfPartMax = size_t{128} << 20;
 // 32-key sub-chunks, and two work-groups share a CU, so the kernel's time is
 // about the larger of its longest work-group and the total work over the
 // resident work-groups.  Blocks longer than a third of the longest (and than
-// 8 sub-chunks) are cut into parts of their key range of at most that
+// 8 sub-chunks; less where the grid is short, below) are cut into parts of their key range of at most that
 // length, each a work-group, whose partial results attn_prefill_merge_kernel
 // combines; grid rows are ordered longest first.  (2048 tokens, 32/8 heads:
 // kernel + merge 200 us per layer unsplit; halves 163 + 12, thirds best,
@@ -1360,6 +1360,7 @@ bool attention_prefill_plan(const PrefillArgs& a, std::vector<int32_t>& tab, int
     std::vector<Item> items;
     std::vector<int32_t> split;
     int32_t maxsub = 0;
+    int64_t work = 0;
     auto range = [&](int32_t blk, int32_t& lo, int32_t& hi) {
         const int32_t q0 = blk * TQ, nq = std::min(TQ, a.batch - q0);
         hi = a.pos0 + q0 + nq - 1;
@@ -1369,16 +1370,25 @@ bool attention_prefill_plan(const PrefillArgs& a, std::vector<int32_t>& tab, int
         int32_t lo, hi;
         range(blk, lo, hi);
         maxsub = std::max(maxsub, (hi - lo) / kPfKeys + 1);
+        work += (hi - lo) / kPfKeys + 1;
     }
     if (maxsub <= 8) return false;
-    const int32_t cut = std::max<int32_t>(8, (maxsub + 2) / 3);
+    // few blocks (a short batch, or one on a long cache) leave CUs idle: parts
+    // short enough to make 384 work-groups, at least 4 sub-chunks, at most
+    // kPfMaxParts of them (whole calls, 32/8 heads, thirds / this: 10 tokens at
+    // position 2000 79.5 / 34.3 us, 64 at 1000 54.9 / 26.8, 300 at 0 47.6 /
+    // 28.6, the prologue's change included; for 512 work-groups 1000 tokens took
+    // 75.7 us against 65.4)
+    const int32_t fill = static_cast<int32_t>((work * a.n_kv_heads + 383) / 384);
+    const int32_t cut = std::min(std::max<int32_t>(8, (maxsub + 2) / 3),
+                                 std::max({4, (maxsub + kPfMaxParts - 1) / kPfMaxParts, fill}));
     int32_t slots = 0;
     for (int32_t blk = nblk - 1; blk >= 0; --blk) {
         int32_t lo, hi;
         range(blk, lo, hi);
         const int32_t nsub = (hi - lo) / kPfKeys + 1;
         if (nsub > cut) {
-            const int32_t parts = (nsub + cut - 1) / cut;  // at most 3 (cut >= maxsub / 3)
+            const int32_t parts = (nsub + cut - 1) / cut;
             if (parts > kPfMaxParts) return false;
             split.insert(split.end(), {blk, slots, parts});
             for (int32_t q = 0; q < parts; ++q) {

@@ -434,6 +434,15 @@ def test_attention_prefill_prologue_bitexact(lib, H, KV, weight, base, off):
     assert np.array_equal(kc1, kc) and np.array_equal(vc1, vc)
 
 
+# short batches on long caches: key ranges in up to eight parts (one block of
+# 32 tokens, one of 4 rows of 32 heads, a window, one head per KV head, and two
+# blocks of unequal length)
+@pytest.mark.parametrize("H,KV,pos0,B,sw", [(32, 8, 1990, 10, 0), (32, 1, 700, 3, 0), (32, 8, 1500, 40, 512),
+                                            (16, 16, 1000, 5, 0), (32, 8, 300, 33, 0)])
+def test_attention_prefill_short_batch_parts(lib, H, KV, pos0, B, sw):
+    test_attention_prefill_equals_fused_steps(lib, H, KV, 128, pos0, B, sw)
+
+
 @pytest.mark.parametrize("pos0,B,sw", [(10, 64, 0), (300, 200, 0), (0, 600, 200)])
 def test_attention_prefill_device_buffers(lib, oracle, pos0, B, sw):
     """Device-resident buffers (used in place), against the oracle's
