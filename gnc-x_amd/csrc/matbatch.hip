@@ -1237,54 +1237,62 @@ __global__ __launch_bounds__(512, 1) void matbatch_bf16_kernel(const uint8_t* __
 }
 
 // y = sum over the split K ranges, added in range order (deterministic);
-// range z's partials are the flat block [z count, (z + 1) count).  The
-// first kRedU ranges are loaded together before the adds (a loop of
-// load-then-add waited on memory once per range).
-constexpr int kRedU = 16;
-
-// V: float, or floatx4 where every output is whole, aligned groups of four
-// (64 x 4096 outputs of 16 ranges: see launch_reduce)
-template <class V>
+// range z's partials are the flat block [z count, (z + 1) count).  Ranges are
+// loaded U at a time, all U loads issued before the first add, without a
+// branch (a range past the last reads the last again and is not added): with a
+// branch around each load, 64 x 4096 outputs of 16 ranges took the call 2.6 us
+// longer.  V: float, a thread per output, or floatx4 for many outputs
+// (launch_reduce).
+template <class V, int U>
 __global__ __launch_bounds__(kThreads) void matbatch_reduce_kernel(const float* __restrict part, int32_t splits,
                                                                    RedMats r) {
     constexpr size_t W = sizeof(V) / sizeof(float);
     const size_t count = r.end[r.count - 1] / W;
     const V* __restrict p = reinterpret_cast<const V*>(part);
-    for (size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x; i < count;
-         i += static_cast<size_t>(gridDim.x) * kThreads) {
-        V v[kRedU];
+    const size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >= count) return;
+    V acc = p[i];
+    for (int32_t z = 1; z < splits; z += U) {
+        V v[U];
 #pragma unroll
-        for (int u = 0; u < kRedU; ++u) v[u] = u < splits ? p[static_cast<size_t>(u) * count + i] : V{};
-        V acc = v[0];
+        for (int u = 0; u < U; ++u) v[u] = p[static_cast<size_t>(min(z + u, splits - 1)) * count + i];
 #pragma unroll
-        for (int u = 1; u < kRedU; ++u)
-            if (u < splits) acc += v[u];
-        for (int32_t z = kRedU; z < splits; ++z) acc += p[static_cast<size_t>(z) * count + i];
-        float* y = r.y[0];
-        size_t first = 0;
-#pragma unroll
-        for (int m = 1; m < kMaxMbMats; ++m) {
-            if (r.count > m && i * W >= r.end[m - 1]) {
-                y = r.y[m];
-                first = r.end[m - 1];
-            }
-        }
-        *reinterpret_cast<V*>(&y[i * W - first]) = acc;
+        for (int u = 0; u < U; ++u)
+            if (z + u < splits) acc += v[u];
     }
+    float* y = r.y[0];
+    size_t first = 0;
+#pragma unroll
+    for (int m = 1; m < kMaxMbMats; ++m) {
+        if (r.count > m && i * W >= r.end[m - 1]) {
+            y = r.y[m];
+            first = r.end[m - 1];
+        }
+    }
+    *reinterpret_cast<V*>(&y[i * W - first]) = acc;
 }
 
+template <class V>
+void launch_reduce_t(const float* part, int32_t splits, const RedMats& r, hipStream_t stream) {
+    const size_t count = r.end[r.count - 1] / (sizeof(V) / sizeof(float));
+    const dim3 g(static_cast<unsigned>((count + kThreads - 1) / kThreads)), t(kThreads);
+    if (splits <= 2) hipLaunchKernelGGL((matbatch_reduce_kernel<V, 1>), g, t, 0, stream, part, splits, r);
+    else if (splits <= 4) hipLaunchKernelGGL((matbatch_reduce_kernel<V, 3>), g, t, 0, stream, part, splits, r);
+    else if (splits <= 8) hipLaunchKernelGGL((matbatch_reduce_kernel<V, 7>), g, t, 0, stream, part, splits, r);
+    else hipLaunchKernelGGL((matbatch_reduce_kernel<V, 15>), g, t, 0, stream, part, splits, r);
+}
+
+// Four outputs per thread from 1.25 * 2^20 outputs (whole, aligned groups of four),
+// where the grid fills the chip either way; below that a thread each.  Whole
+// calls, four / one: Q6_K K = 2048, 128 x 4096 27.3 / 21.9 us, 200 x 4096 29.4 /
+// 25.2, 300 x 4096 35.8 / 33.0; Q4_K K = 4096, 64 x 4096 21.0 / 18.2, 512 x
+// 2560 38.5 / 39.1, 1000 x 2048 48.7 / 49.4; Q8_0, 1000 x 2048 61.3 / 62.7.
 hipError_t launch_reduce(const float* part, int32_t splits, const RedMats& r, hipStream_t stream) {
-    bool four = (reinterpret_cast<uintptr_t>(part) & 15u) == 0;
+    bool four = r.end[r.count - 1] >= (size_t{5} << 18) && (reinterpret_cast<uintptr_t>(part) & 15u) == 0;
     for (int32_t i = 0; i < r.count; ++i)
         four = four && r.end[i] % 4 == 0 && (reinterpret_cast<uintptr_t>(r.y[i]) & 15u) == 0;
-    const size_t count = r.end[r.count - 1] / (four ? 4 : 1);
-    const size_t g = std::min<size_t>((count + kThreads - 1) / kThreads, 4096);
-    if (four)
-        hipLaunchKernelGGL(matbatch_reduce_kernel<floatx4>, dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, stream,
-                           part, splits, r);
-    else
-        hipLaunchKernelGGL(matbatch_reduce_kernel<float>, dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, stream,
-                           part, splits, r);
+    if (four) launch_reduce_t<floatx4>(part, splits, r, stream);
+    else launch_reduce_t<float>(part, splits, r, stream);
     return hipGetLastError();
 }
 

@@ -376,6 +376,26 @@ def test_matbatch_stream_tiles(lib, oracle, t, k, n, b):
     assert rel_l2(y, want) < 5e-7
 
 
+# The split-K reduce: its number of ranges (1 + a multiple of the 1, 3, 7 or 15
+# that a thread loads at a time, and around it), odd output counts, and from
+# 1.25 * 2^20 outputs four per thread (aligned groups) or, N odd, one.
+REDUCE_CASES = [(256 * s, 33, 5) for s in (3, 4, 5, 8, 9, 16, 17, 31, 57)] + [
+    (1024, 4097, 130), (1024, 2048, 640), (1024, 2561, 512), (768, 3000, 300)]  # 4, 2, 2 and 3 ranges
+
+
+@pytest.mark.parametrize("k,n,b", REDUCE_CASES)
+def test_matbatch_split_reduce(lib, oracle, k, n, b):
+    w = synth.make_weights(Q4_K, n, k, seed=3200 + k + n)
+    x = synth.make_activations(b, k, seed=4200 + k + b).reshape(b, k)
+    y = np.full((b, n), np.nan, np.float32)
+    lib.gncx_xfold_universal_matbatch(ptr(w), 0, Q4_K, ptr(x), b, k, n, ptr(y), None)
+    gncx.check(lib)
+    want = oracle.matbatch(Q4_K, w, x, b, k, n)
+    # K / 256 super-blocks, each exact up to 8 + 2 roundings of 2^-24 of its
+    # terms, random in sign, in any split; a range lost or added twice is 2 / 57
+    assert rel_l2(y, want) < 5e-7
+
+
 # Q6_K scales beyond +-64 (real quantisers use the whole int8 range): then
 # sc (q - 32) can exceed 2048 and the 256-token tiles add the third product in
 # the steps that hold such a scale.  All rows large, none, and one row in
