@@ -359,8 +359,9 @@ struct RedMats {
 // ahead; nothing about the weights goes through LDS but the rows' scales.
 // One v_mfma_f32_16x16x32_f16 is one 32-value block of a 16 x 16 tile: lane
 // l holds row (A operand, weights) or token (B, activations) l % 16 and
-// values 8 g .. 8 g + 7 of the block, g = l / 16, in the order 0 2 1 3 4 6 5
-// 7 on both sides (the order in which masks pick byte pairs out of a dword).
+// values 8 kg .. 8 kg + 7 of the block, kg = kgroup(l / 16) (0 2 1 3), in the
+// order 0 2 1 3 4 6 5 7 (the order in which masks pick byte pairs out of a
+// dword), on both sides.
 // Weights are small integers, exact in fp16, and activations the quantised q,
 // so a block's product is its exact integer dot (below 2^24).  The block
 // scales are applied on the VALU: S += (d_x / s) dot, where d of Q8_0 / Q4_0
@@ -400,81 +401,184 @@ __device__ __forceinline__ half2 h2_of(uint32_t v) { return __builtin_bit_cast(h
 __device__ __forceinline__ uint32_t u_of(half2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ half2 h2_all(float v) { return half2{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
 
-// One super-block of a lane's weight row in registers: the bytes that hold
-// its 8 values of each block, and the scales.  A register is loaded again,
-// for the next super-block, as soon as its last block's operands are formed:
-// load<P>(byte offset, lane group g, further blocks of the row) issues the
-// loads of part P, -1 for the scales and j for what block j uses last.
-// Blocks past the row (Q8_0, Q4_0: nblk) read zeros.
-template <int TYPE>
+// One super-block of a lane's weight row in registers.  A load costs the
+// address path a cycle per lane, whatever its width (lanes of different rows
+// share no line), which is what bounds the tiles of 16 and 32 tokens: so 16
+// bytes a load, not the 8 that one block's operand takes of a row.  One
+// work-group of 256 Q4_K rows per CU, loads alone: 2.25 -> 1.40 us per
+// super-block; whole calls of 4096 x 4096 at B = 11, Q4_K 13.7 -> 12.7 us, Q8_0
+// 18.6 -> 17.9, of 4096 x 14336 at B = 64, Q8_0 49.2 -> 45.0, Q4_0 46.0 -> 42.0.
+// A 16-byte load holds two 8-byte pieces of a 32-byte run of the row, and four
+// lane groups two runs A, B (Q4_K: two sub-block pairs): A01 A23 B01 B23.
+// settle() exchanges the upper halves of lanes 0-31 with the lower halves of
+// lanes 32-63: A0 A2 A1 A3 in x, y and B0 B2 B1 B3 in z, w.  So lane group g
+// holds values 8 kg .. of each block, kg = kgroup(g), and reads the
+// activations in that order.
+// A register is loaded again, for the next super-block, as soon as its last
+// block's operands are formed: load<P>(byte offset, lane group g, blocks left
+// in the row) issues the loads of part P, of what block P uses last (-1: of
+// what is used first).  begin(j) settles what block j is the first to use, and
+// at(j, d) is dword d of its bytes.  Blocks past the row (Q8_0, Q4_0: nblk)
+// read zeros.
+__device__ __forceinline__ int kgroup(int g) { return (g >> 1) | ((g & 1) << 1); }
+__device__ __forceinline__ void settle(u32x4& q) {
+    const auto a = __builtin_amdgcn_permlane32_swap(q.x, q.z, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(q.y, q.w, false, false);
+    q = u32x4{a[0], b[0], a[1], b[1]};
+}
+__device__ __forceinline__ uint32_t dword_of(const u32x4& q, int i) {
+    return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w;
+}
+// WIDE (kQsWide): where it measured faster.  Two blocks a load hold registers
+// longer: at 128 tokens Q8_0 spilled (8-18% slower) and Q4_0 (1-5%); Q6_K from
+// 64 tokens is slower on rows of 2-byte alignment (2816 x 5000 at B = 2048 194
+// -> 203 us, with 8-byte loads 195).
+template <int TYPE, int TF>
+constexpr bool kQsWide = TYPE == kQ6_K ? TF < 4 : TF < 8;
+template <int TYPE, bool WIDE>
 struct QsW;
-template <>
-struct QsW<kQ4_K> {
-    static constexpr int32_t kBytes = 144;
-    static constexpr int kLoads = 5;
-    u32x4 h;
-    u32x2 q[4];  // bytes 8 g .. of each sub-block pair's 32
+template <bool WIDE>
+struct QsW<kQ4_K, WIDE> {
+    static constexpr int kLoads = 2;
+    u32x4 q[2];  // sub-block pairs 2 i and 2 i + 1
     template <int P>
     __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t) {
-        if constexpr (P == -1) h = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-        else if constexpr ((P & 1) == 1)
-            q[P >> 1] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 16 + 16 * (P - 1), 0, 0);
+        if constexpr (P >= 0 && (P & 3) == 3)
+            q[P >> 2] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 + 64 * (P >> 2) + 16 * g, 0, 0);
     }
+    __device__ __forceinline__ void begin(int j) {
+        if ((j & 3) == 0) settle(q[j >> 2]);
+    }
+    __device__ __forceinline__ uint32_t at(int j, int d) const { return dword_of(q[j >> 2], (j & 2) + d); }
 };
 template <>
-struct QsW<kQ6_K> {
-    static constexpr int32_t kBytes = 210;
-    static constexpr int kLoads = 8;
-    u32x4 s;           // the 16 scales
-    u32x2 l[4], u[2];  // ql bytes 8 g .. of each 32, qh bytes 8 g .. of each 32
-    uint32_t d;
+struct QsW<kQ6_K, true> {
+    static constexpr int kLoads = 4;
+    u32x4 l[2];  // ql of half i: its first and second 32 bytes
+    u32x2 u[2];  // qh bytes 8 kg .. of half i (16 bytes of both would fall free with block 7 only)
     template <int P>
     __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t) {
-        if constexpr (P == -1) {
-            s = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 192, 0, 0);
-            d = __builtin_amdgcn_raw_buffer_load_b16(rs, off + 208, 0, 0);
-        } else if constexpr ((P & 2) == 2) {
-            constexpr int i = 2 * (P >> 2) + (P & 1);
-            l[i] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 32 * i, 0, 0);
-            if constexpr ((P & 1) == 1)
-                u[P >> 2] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * g + 128 + 32 * (P >> 2), 0, 0);
+        if constexpr (P >= 0 && (P & 3) == 3) {
+            l[P >> 2] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 64 * (P >> 2) + 16 * g, 0, 0);
+            u[P >> 2] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 128 + 32 * (P >> 2) + 8 * kgroup(g), 0, 0);
         }
     }
+    __device__ __forceinline__ void begin(int j) {
+        if ((j & 3) == 0) settle(l[j >> 2]);
+    }
+    __device__ __forceinline__ uint32_t at(int j, int d) const { return dword_of(l[j >> 2], 2 * (j & 1) + d); }
+    __device__ __forceinline__ uint32_t up(int j, int d) const { return d == 0 ? u[j >> 2].x : u[j >> 2].y; }
 };
 template <>
-struct QsW<kQ8_0> {
-    static constexpr int32_t kBytes = 272;
+struct QsW<kQ6_K, false> {
+    static constexpr int kLoads = 6;
+    u32x2 l[4], u[2];  // ql bytes 8 kg .. of each 32, qh bytes 8 kg .. of each 32
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t) {
+        if constexpr (P >= 0 && (P & 2) == 2) {
+            constexpr int i = 2 * (P >> 2) + (P & 1);
+            l[i] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * kgroup(g) + 32 * i, 0, 0);
+            if constexpr ((P & 1) == 1)
+                u[P >> 2] = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 8 * kgroup(g) + 128 + 32 * (P >> 2), 0, 0);
+        }
+    }
+    __device__ __forceinline__ void begin(int) {}
+    __device__ __forceinline__ uint32_t at(int j, int d) const {
+        const u32x2 v = l[2 * (j >> 2) + (j & 1)];
+        return d == 0 ? v.x : v.y;
+    }
+    __device__ __forceinline__ uint32_t up(int j, int d) const { return d == 0 ? u[j >> 2].x : u[j >> 2].y; }
+};
+// Q8_0 and Q4_0 (BB bytes a block): the scales of blocks 2 g and 2 g + 1
+template <int BB>
+struct QsBlockScales {
+    uint32_t d[2];
+    __device__ __forceinline__ void load_d(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            d[e] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * g + e < nblk ? off + BB * (2 * g + e) : kMfOob, 0, 0);
+    }
+};
+// wide: blocks 2 i and 2 i + 1 in q[i].  Q4_0: bytes 8 (g / 2) .. of a block's
+// 16, of which lane group g takes the low (g even) or high nibbles, which are
+// values 8 kg .. again
+template <int BB>
+struct QsWideBlocks : QsBlockScales<BB> {
+    static constexpr int kLoads = 6;
+    u32x4 q[4];
+    template <int P>
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
+        if constexpr (P == -1) this->load_d(rs, off, g, nblk);
+        else if constexpr ((P & 1) == 1) {
+            const int blk = P - 1 + (g >> 1), at = BB == 34 ? 16 * (g & 1) : 0;
+            q[P >> 1] = __builtin_amdgcn_raw_buffer_load_b128(rs, blk < nblk ? off + BB * blk + 2 + at : kMfOob, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void begin(int j) {
+        if ((j & 1) == 0) settle(q[j >> 1]);
+    }
+    __device__ __forceinline__ uint32_t at(int j, int d) const { return dword_of(q[j >> 1], 2 * (j & 1) + d); }
+};
+// one block's 8 bytes a load
+template <int BB>
+struct QsNarrowBlocks : QsBlockScales<BB> {
     static constexpr int kLoads = 10;
     u32x2 q[8];
-    uint32_t d[2];  // of blocks 2 g and 2 g + 1
     template <int P>
     __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
-        if constexpr (P == -1) {
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-                d[e] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * g + e < nblk ? off + 34 * (2 * g + e) : kMfOob, 0, 0);
-        } else {
-            q[P] = __builtin_amdgcn_raw_buffer_load_b64(rs, P < nblk ? off + 8 * g + 34 * P + 2 : kMfOob, 0, 0);
+        if constexpr (P == -1) this->load_d(rs, off, g, nblk);
+        else {
+            const int at = BB == 34 ? 8 * kgroup(g) : 8 * (g >> 1);
+            q[P] = __builtin_amdgcn_raw_buffer_load_b64(rs, P < nblk ? off + BB * P + 2 + at : kMfOob, 0, 0);
         }
+    }
+    __device__ __forceinline__ void begin(int) {}
+    __device__ __forceinline__ uint32_t at(int j, int d) const { return d == 0 ? q[j].x : q[j].y; }
+};
+template <>
+struct QsW<kQ8_0, true> : QsWideBlocks<34> {};
+template <>
+struct QsW<kQ8_0, false> : QsNarrowBlocks<34> {};
+template <>
+struct QsW<kQ4_0, true> : QsWideBlocks<18> {};
+template <>
+struct QsW<kQ4_0, false> : QsNarrowBlocks<18> {};
+
+// The super-block scales of both fragments' rows, one load for the wave (as
+// above): lane l reads row l % 32, row l % 16 of fragment l / 16 % 2, and
+// spread() gives every lane the scales of its row of each fragment, odd lane
+// groups of one copy exchanged with even ones of another.
+template <int TYPE>
+struct QsH {  // Q8_0, Q4_0: the block scales are in QsW
+    static constexpr int kLoads = 0;
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t&, int32_t) {}
+};
+template <>
+struct QsH<kQ4_K> {
+    static constexpr int kLoads = 1;
+    u32x4 h;  // d and dmin, the 12 scale bytes
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off) {
+        h = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
     }
 };
 template <>
-struct QsW<kQ4_0> {
-    static constexpr int32_t kBytes = 144;
-    static constexpr int kLoads = 10;
-    u32x2 q[8];  // bytes 8 (g % 2) .. of each block's 16
-    uint32_t d[2];
-    template <int P>
-    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off, int g, int32_t nblk) {
-        if constexpr (P == -1) {
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-                d[e] = __builtin_amdgcn_raw_buffer_load_b16(rs, 2 * g + e < nblk ? off + 18 * (2 * g + e) : kMfOob, 0, 0);
-        } else {
-            q[P] = __builtin_amdgcn_raw_buffer_load_b64(rs, P < nblk ? off + 8 * (g & 1) + 18 * P + 2 : kMfOob, 0, 0);
-        }
+struct QsH<kQ6_K> {
+    static constexpr int kLoads = 2;
+    u32x4 h;  // the 16 scales
+    uint32_t d;
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& rs, int32_t off) {
+        h = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 192, 0, 0);
+        d = __builtin_amdgcn_raw_buffer_load_b16(rs, off + 208, 0, 0);
     }
 };
+__device__ __forceinline__ void spread(const u32x4& h, u32x4 (&o)[2]) {
+    const auto x = __builtin_amdgcn_permlane16_swap(h.x, h.x, false, false);
+    const auto y = __builtin_amdgcn_permlane16_swap(h.y, h.y, false, false);
+    const auto z = __builtin_amdgcn_permlane16_swap(h.z, h.z, false, false);
+    const auto w = __builtin_amdgcn_permlane16_swap(h.w, h.w, false, false);
+    o[0] = u32x4{x[0], y[0], z[0], w[0]};
+    o[1] = u32x4{x[1], y[1], z[1], w[1]};
+}
 
 // (v & mask) | e as one v_and_or_b32: with e hidden in a vector register and
 // the mask in a scalar one (two literals would take two instructions)
@@ -483,9 +587,10 @@ __device__ __forceinline__ uint32_t in_vgpr(uint32_t v) {
     return v;
 }
 
-// The A operands of a lane's row for one super-block: prepare() unpacks what
-// all blocks share, get(w, g, j, d, o) forms dword d (0, 1) of block j's
-// operand, 4 of its 8 values (o.b: Q6_K's second product).
+// The A operands of a lane's row for one super-block: prepare(h, g) unpacks
+// what all blocks share from the row's scales, get(w, g, j, d, o) forms dword d
+// (0, 1; 0 first) of block j's operand, 4 of its 8 values (o.b: Q6_K's second
+// product).
 struct QsOut {
     uint32_t a[4], b[4];
 };
@@ -496,15 +601,17 @@ struct QsOperand<kQ4_K> {
     uint32_t sc[2], mn[2];  // 6-bit scales and mins of sub-blocks 0-3 and 4-7, a byte each
     uint32_t e;
     half2 s, m;  // of the block being formed
-    __device__ __forceinline__ void prepare(const QsW<kQ4_K>& w, int) {
+    __device__ __forceinline__ void prepare(const u32x4& h, int) {
         e = in_vgpr(0x64006400u);
-        sc[0] = w.h.y & 0x3f3f3f3fu;
-        mn[0] = w.h.z & 0x3f3f3f3fu;
-        sc[1] = (w.h.w & 0x0f0f0f0fu) | ((w.h.y >> 2) & 0x30303030u);
-        mn[1] = ((w.h.w >> 4) & 0x0f0f0f0fu) | ((w.h.z >> 2) & 0x30303030u);
+        sc[0] = h.y & 0x3f3f3f3fu;
+        mn[0] = h.z & 0x3f3f3f3fu;
+        sc[1] = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+        mn[1] = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
     }
-    __device__ __forceinline__ void get(const QsW<kQ4_K>& w, int, int j, int d, QsOut& o) {
+    template <class W>
+    __device__ __forceinline__ void get(W& w, int, int j, int d, QsOut& o) {
         if (d == 0) {
+            w.begin(j);
             const uint32_t sel = 0x04000400u | (0x00010001u * static_cast<uint32_t>(j & 3));
             const half2 t = h2_of(__builtin_amdgcn_perm(0x64646464u, sc[j >> 2], sel));  // 1024 + sc
             // low nibbles sit under the exponent of 1024 as they are, high ones times 16
@@ -512,7 +619,7 @@ struct QsOperand<kQ4_K> {
             m = s * h2_all(-1024.0f);
         }
         const uint32_t mask = (j & 1) == 0 ? 0x000f000fu : 0x00f000f0u;
-        const uint32_t v = d == 0 ? w.q[j >> 1].x : w.q[j >> 1].y;
+        const uint32_t v = w.at(j, d);
         o.a[2 * d] = u_of(__builtin_elementwise_fma(h2_of((v & mask) | e), s, m));
         o.a[2 * d + 1] = u_of(__builtin_elementwise_fma(h2_of(((v >> 8) & mask) | e), s, m));
     }
@@ -522,24 +629,24 @@ struct QsOperand<kQ6_K> {
     uint32_t sc[4];  // scale + 128 of blocks 2 i and 2 i + 1 in bytes 0 and 2
     uint32_t e1, e2;
     half2 s1, m1, s2, m2;
-    __device__ __forceinline__ void prepare(const QsW<kQ6_K>& w, int g) {
+    __device__ __forceinline__ void prepare(const u32x4& h, int g) {
         e1 = in_vgpr(0x4c004c00u);
         e2 = in_vgpr(0x44004400u);
-        const uint32_t v[4] = {w.s.x, w.s.y, w.s.z, w.s.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sc[i] = (v[i] ^ 0x80808080u) >> (8 * (g >> 1));
+        for (int i = 0; i < 4; ++i) sc[i] = (dword_of(h, i) ^ 0x80808080u) >> (8 * (kgroup(g) >> 1));
     }
-    __device__ __forceinline__ void get(const QsW<kQ6_K>& w, int, int j, int d, QsOut& o) {
-        const int hf = j >> 2, gr = j & 3;
+    template <class W>
+    __device__ __forceinline__ void get(W& w, int, int j, int d, QsOut& o) {
+        const int gr = j & 3;
         if (d == 0) {
+            w.begin(j);
             const uint32_t sel = (j & 1) == 0 ? 0x04000400u : 0x04020402u;
             s1 = h2_of(__builtin_amdgcn_perm(0x64646464u, sc[j >> 1], sel)) + h2_all(-1152.0f);
             m1 = s1 * h2_all(-32.0f);
             s2 = s1 * h2_all(16.0f);
             m2 = s1 * h2_all(-80.0f);
         }
-        const u32x2 lv = w.l[2 * hf + (gr & 1)], uv = w.u[hf];
-        const uint32_t l = d == 0 ? lv.x : lv.y, u = d == 0 ? uv.x : uv.y;
+        const uint32_t l = w.at(j, d), u = w.up(j, d);
         // the nibbles of bytes 0, 2 / 1, 3 at bits 6..9 of each half: 16 + l
         const uint32_t l0 = gr < 2 ? l << 6 : l << 2, l1 = gr < 2 ? l >> 2 : l >> 6;
         o.a[2 * d] = u_of(__builtin_elementwise_fma(h2_of((l0 & 0x03c003c0u) | e1), s1, m1));
@@ -552,19 +659,23 @@ struct QsOperand<kQ6_K> {
 };
 template <>
 struct QsOperand<kQ8_0> {
-    __device__ __forceinline__ void prepare(const QsW<kQ8_0>&, int) {}
-    __device__ __forceinline__ void get(const QsW<kQ8_0>& w, int, int j, int d, QsOut& o) {
-        const uint32_t v = (d == 0 ? w.q[j].x : w.q[j].y) ^ 0x80808080u;  // q + 128 per byte
+    __device__ __forceinline__ void prepare(const u32x4&, int) {}
+    template <class W>
+    __device__ __forceinline__ void get(W& w, int, int j, int d, QsOut& o) {
+        if (d == 0) w.begin(j);
+        const uint32_t v = w.at(j, d) ^ 0x80808080u;  // q + 128 per byte
         o.a[2 * d] = u_of(h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)) + h2_all(-1152.0f));
         o.a[2 * d + 1] = u_of(h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)) + h2_all(-1152.0f));
     }
 };
 template <>
 struct QsOperand<kQ4_0> {
-    __device__ __forceinline__ void prepare(const QsW<kQ4_0>&, int) {}
-    __device__ __forceinline__ void get(const QsW<kQ4_0>& w, int g, int j, int d, QsOut& o) {
+    __device__ __forceinline__ void prepare(const u32x4&, int) {}
+    template <class W>
+    __device__ __forceinline__ void get(W& w, int g, int j, int d, QsOut& o) {
+        if (d == 0) w.begin(j);
         // values 0-15 are the low nibbles of the 16 bytes, 16-31 the high ones
-        const uint32_t v = (d == 0 ? w.q[j].x : w.q[j].y) >> (4 * (g >> 1));
+        const uint32_t v = w.at(j, d) >> (4 * (kgroup(g) >> 1));
         o.a[2 * d] = u_of(h2_of((v & 0x000f000fu) | 0x64006400u) + h2_all(-1032.0f));
         o.a[2 * d + 1] = u_of(h2_of(((v >> 8) & 0x000f000fu) | 0x64006400u) + h2_all(-1032.0f));
     }
@@ -646,25 +757,28 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     // this lane's weight rows, 32 wv + 16 f + l % 16; rows past N and
     // super-blocks past the range read zeros (offsets past the resource,
     // whose base is the dword at or below the first row)
-    constexpr int32_t kWB = QsW<TYPE>::kBytes;
+    using W = QsW<TYPE, kQsWide<TYPE, TF>>;
+    using H = QsH<TYPE>;
+    constexpr int32_t kWB = TYPE == kQ6_K ? 210 : TYPE == kQ8_0 ? 272 : 144;  // bytes of a super-block
     const uint8_t* wt = w + static_cast<size_t>(n0) * rbytes;
     const int32_t delta = TYPE == kQ4_K ? 0 : static_cast<int32_t>(reinterpret_cast<uintptr_t>(wt) & 3u);
     const __amdgpu_buffer_rsrc_t wrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wt - delta), static_cast<short>(0),
                                           wrows_here * static_cast<int32_t>(rbytes) + delta, 0x00020000);
-    int32_t wbase[RF];
-#pragma unroll
-    for (int f = 0; f < RF; ++f) {
-        const int32_t row = 32 * wv + 16 * f + l16;
-        wbase[f] = row < wrows_here ? row * static_cast<int32_t>(rbytes) + delta + kb / 256 * kWB : kMfOob / 2;
-    }
+    auto row_at = [&](int32_t row) {
+        return row < wrows_here ? row * static_cast<int32_t>(rbytes) + delta + kb / 256 * kWB : kMfOob / 2;
+    };
+    const int32_t wbase[RF] = {row_at(32 * wv + l16), row_at(32 * wv + 16 + l16)};
+    const int32_t hbase = row_at(32 * wv + (lane & 31));
     struct SbRegs {
-        QsW<TYPE> f[RF];
+        H h;
+        W f[RF];
     };
     SbRegs R;
     // part P of super-block s
     auto wload = [&]<int P>(std::integral_constant<int, P>, int32_t s) {
         const int32_t nblk = SUPER ? 8 : (ke - kb - 256 * s) / 32, at = s < nsb ? s * kWB : kMfOob / 2;
+        if constexpr (P == -1) R.h.load(wrs, hbase + at);
 #pragma unroll
         for (int f = 0; f < RF; ++f) R.f[f].template load<P>(wrs, wbase[f] + at, lg, nblk);
     };
@@ -715,7 +829,7 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     constexpr int kXLoads = kXQ + kXP * (TYPE == kQ4_K ? 2 : 1);
     // the loads that may be in flight past a super-block's barrier: its own
     // (weights of the next one and, with three stages, activations two ahead)
-    constexpr int kLoads = RF * QsW<TYPE>::kLoads + (S3 ? kXLoads : 0);
+    constexpr int kLoads = H::kLoads + RF * W::kLoads + (S3 ? kXLoads : 0);
     auto wfirst = [&] {
         [&]<int... P>(std::integer_sequence<int, P...>) {
             (wload(std::integral_constant<int, P - 1>{}, 0), ...);
@@ -749,17 +863,18 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     // loaded as the registers fall free
     auto process = [&](const _Float16* xst, const float* sdt, const _Float16* spt, int32_t s) {
         QsOperand<TYPE> op[RF];
+        u32x4 hf[RF] = {};
+        if constexpr (SUPER) spread(R.h.h, hf);
 #pragma unroll
-        for (int f = 0; f < RF; ++f) op[f].prepare(R.f[f], lg);
+        for (int f = 0; f < RF; ++f) op[f].prepare(hf[f], lg);
         // the accumulator rows' scales, exchanged through LDS within the wave
         if constexpr (TYPE == kQ4_K) {
-            if (lg < 2) {
-                const uint32_t h = lg == 0 ? R.f[0].h.x : R.f[1].h.x;
-                sdm[wv][0][16 * lg + l16] = half_bits_to_float(h & 0xffffu);
-                sdm[wv][1][16 * lg + l16] = half_bits_to_float(h >> 16);
+            if (lane < 32) {
+                sdm[wv][0][lane] = half_bits_to_float(R.h.h.x & 0xffffu);
+                sdm[wv][1][lane] = half_bits_to_float(R.h.h.x >> 16);
             }
         } else if constexpr (TYPE == kQ6_K) {
-            if (lg < 2) sdm[wv][0][16 * lg + l16] = half_bits_to_float(lg == 0 ? R.f[0].d : R.f[1].d);
+            if (lane < 32) sdm[wv][0][lane] = half_bits_to_float(R.h.d);
         } else {
 #pragma unroll
             for (int f = 0; f < RF; ++f)
@@ -769,7 +884,7 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
         wload(std::integral_constant<int, -1>{}, s + 1);
         // LDS offsets; hidden from the compiler, which would otherwise keep
         // one register per block for each across the loop
-        int xa = 256 * l16 + 8 * (lg ^ l16), da = 8 * l16 + (l16 >> 2);
+        int xa = 256 * l16 + 8 * (kgroup(lg) ^ l16), da = 8 * l16 + (l16 >> 2);
         asm volatile("" : "+v"(xa), "+v"(da));
         auto x_at = [&](int j, int t) {
             return *reinterpret_cast<const half8*>(&xst[(xa ^ (32 * j)) + 4096 * t]);

@@ -376,6 +376,26 @@ def test_matbatch_stream_tiles(lib, oracle, t, k, n, b):
     assert rel_l2(y, want) < 5e-7
 
 
+# The streamed kernel's steady state on each tile: whole K per work-group (no
+# range is shorter than these), 5 super-blocks of Q4_K and Q6_K and 4 and one
+# block of Q4_0 and Q8_0, so that every stage and register is refilled, the
+# weights of a super-block follow those of another, the last one is partly past
+# the row, and the loads past the end are in flight at the output.  (B, N):
+# 16-, 32-, 64- and 128-token tiles, ragged in both.
+@pytest.mark.parametrize("t,k", [(Q4_0, 1056), (Q8_0, 1056), (Q4_K, 1280), (Q6_K, 1280)])
+@pytest.mark.parametrize("n,b", [(40001, 9), (40001, 30), (40001, 50), (20001, 300)])
+def test_matbatch_stream_steady_state(lib, oracle, t, k, n, b):
+    w = synth.make_weights(t, n, k, seed=3300 + t + b)
+    x = synth.make_activations(b, k, seed=4300 + t + b).reshape(b, k)
+    y = np.full((b, n), np.nan, np.float32)
+    try:
+        lib.gncx_xfold_universal_matbatch(ptr(w), 0, t, ptr(x), b, k, n, ptr(y), None)
+        gncx.check(lib)
+    finally:
+        lib.gncx_hip_weight_forget(ptr(w))
+    assert rel_l2(y, oracle.matbatch(t, w, x, b, k, n)) < 5e-7  # exact block dots, as above
+
+
 # The split-K reduce: its number of ranges (1 + a multiple of the 1, 3, 7 or 15
 # that a thread loads at a time, and around it), odd output counts, and from
 # 1.25 * 2^20 outputs four per thread (aligned groups) or, N odd, one.
