@@ -310,10 +310,10 @@ constexpr int32_t kMfOob = 0x7ff00000;
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
 // vmcnt(N) and lgkmcnt(0), then a work-group barrier with no memory fence.
-// __syncthreads() also waits for the direct-to-LDS loads issued for later
-// steps (its release fence covers every outstanding write, those included),
-// which put a memory round trip on every step.  Here each wave waits only for
-// the loads the next step reads (vmcnt(N)) and for its own LDS writes
+// __syncthreads() says nothing of direct-to-LDS loads: in the loop the compiler
+// waited there for those of later steps too (a memory round trip on every
+// step), at the output of some instances for none.  Here each wave waits only
+// for the loads the next step reads (vmcnt(N)) and for its own LDS writes
 // (lgkmcnt(0)) before the barrier, so after it every wave sees both; the
 // empty asm statements keep the compiler from moving LDS accesses across it.
 template <int N>
@@ -1055,8 +1055,10 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     }
 #undef GNCX_QS_STEP
 
-    // the tile as [token][BN + 4] floats in LDS, then whole token rows out
-    __syncthreads();
+    // the tile as [token][BN + 4] floats in LDS, then whole token rows out;
+    // first the loads past the range, which write zeros into a stage and which
+    // __syncthreads() does not wait for by itself
+    step_barrier<0>();
     constexpr int HT = BM / 2;  // tokens per stage array
 #pragma unroll
     for (int t = 0; t < TF; ++t) {
