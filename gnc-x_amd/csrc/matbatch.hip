@@ -1629,7 +1629,9 @@ hipError_t launch_matbatch(int32_t type, const uint8_t* w, const float* x, int32
     if (k <= 0 || k > (1 << 20) || b > 65535) return hipErrorInvalidValue;  // keeps buffer offsets in int32
     if (type != kBF16 && (k % 32) != 0) return hipErrorInvalidValue;
     if ((type == kQ4_K || type == kQ6_K) && (k % 256) != 0) return hipErrorInvalidValue;
-    if (workspace_bytes < matbatch_workspace_bytes(type, b, k, n)) return hipErrorInvalidValue;
+    const QsPlan p = type == kBF16 ? QsPlan{} : qs_plan(type, b, k, n);
+    const size_t need = type == kBF16 ? matbatch_workspace_bytes(type, b, k, n) : qs_bytes(type, b, k, n, p.splits);
+    if (workspace_bytes < need) return hipErrorInvalidValue;
     const uintptr_t wa = reinterpret_cast<uintptr_t>(w);
     if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0) return hipErrorInvalidValue;
     if (type == kQ4_K || type == kBF16) {
@@ -1650,7 +1652,7 @@ hipError_t launch_matbatch(int32_t type, const uint8_t* w, const float* x, int32
     m.y[0] = y;
     m.n[0] = n;
     m.count = 1;
-    return launch_qs(type, m, q, b, k, qs_plan(type, b, k, n), stream);
+    return launch_qs(type, m, q, b, k, p, stream);
 }
 
 namespace {
@@ -1664,22 +1666,20 @@ bool multi_fused(int32_t type, int32_t count, const int32_t* ns, int32_t b, int3
     total = 0;
     for (int32_t i = 0; i < count; ++i) total += ns[i];
     if (total > INT32_MAX) return false;
-    p = qs_plan(type, b, k, static_cast<int32_t>(total));
     for (int32_t i = 0; i < count; ++i)
         if (ns[i] % kQsRows != 0) return false;
+    p = qs_plan(type, b, k, static_cast<int32_t>(total));
     return true;
 }
 
 }  // namespace
 
 size_t matbatch_multi_workspace_bytes(int32_t type, int32_t count, const int32_t* ns, int32_t b, int32_t k) {
-    size_t need = 256;
-    for (int32_t i = 0; i < count; ++i) need = std::max(need, matbatch_workspace_bytes(type, b, k, ns[i]));
     QsPlan p;
     int64_t total;
-    if (multi_fused(type, count, ns, b, k, p, total)) {
-        need = std::max(need, qs_bytes(type, b, k, total, p.splits));
-    }
+    if (multi_fused(type, count, ns, b, k, p, total)) return qs_bytes(type, b, k, total, p.splits);
+    size_t need = 256;
+    for (int32_t i = 0; i < count; ++i) need = std::max(need, matbatch_workspace_bytes(type, b, k, ns[i]));
     return need;
 }
 
@@ -1689,10 +1689,10 @@ hipError_t launch_matbatch_multi(int32_t type, int32_t count, const uint8_t* con
     if (count <= 0 || count > kMaxMbMats || !ws || !ns || !ys) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
         if (ns[i] <= 0 || !ws[i] || !ys[i]) return hipErrorInvalidValue;
-    if (workspace_bytes < matbatch_multi_workspace_bytes(type, count, ns, b, k)) return hipErrorInvalidValue;
     QsPlan p;
     int64_t total;
     if (!multi_fused(type, count, ns, b, k, p, total)) {
+        if (workspace_bytes < matbatch_multi_workspace_bytes(type, count, ns, b, k)) return hipErrorInvalidValue;
         for (int32_t i = 0; i < count; ++i) {
             const hipError_t e = launch_matbatch(type, ws[i], x, b, k, ns[i], ys[i], workspace, workspace_bytes, stream);
             if (e != hipSuccess) return e;
@@ -1700,6 +1700,7 @@ hipError_t launch_matbatch_multi(int32_t type, int32_t count, const uint8_t* con
         return hipSuccess;
     }
     // the checks of launch_matbatch for Q4_K
+    if (workspace_bytes < qs_bytes(type, b, k, total, p.splits)) return hipErrorInvalidValue;
     if (k > (1 << 20) || b > 65535) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0 || (row_bytes(kQ4_K, k) & 15u) != 0) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
@@ -1729,7 +1730,7 @@ hipError_t launch_matbatch_multi_norm(int32_t type, int32_t count, const uint8_t
     QsPlan p;
     int64_t total;
     if (!multi_fused(type, count, ns, b, k, p, total) || !norm_act_fits(h, r, gamma, k)) return hipErrorNotSupported;
-    if (workspace_bytes < matbatch_multi_workspace_bytes(type, count, ns, b, k)) return hipErrorInvalidValue;
+    if (workspace_bytes < qs_bytes(type, b, k, total, p.splits)) return hipErrorInvalidValue;
     if (k > (1 << 20) || b > 65535 || (row_bytes(kQ4_K, k) & 15u) != 0) return hipErrorInvalidValue;
     for (int32_t i = 0; i < count; ++i)
         if ((reinterpret_cast<uintptr_t>(ws[i]) & 15u) != 0) return hipErrorInvalidValue;
