@@ -1127,7 +1127,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // bf16 parts of 8 values: truncated top 16 bits, the remainder again, and the
 // rest (exact: at most 8 significant bits are left).  Infinite or NaN values
-// leave NaN in the lower parts (the epilogue's check).
+// leave NaN in the lower parts (the output stage's check; zeros below an
+// infinite value, which then needed no check, cost 2-3% on finite ones).
 __device__ __forceinline__ void split3(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
     uint32_t ho[4], mo[4], lo[4];
 #pragma unroll
@@ -1308,35 +1309,59 @@ __global__ __launch_bounds__(512, 1) void matbatch_bf16_kernel(const uint8_t* __
     }
     fold();
 
-    // Infinite and NaN inputs: the parts of an infinite x and the products of
-    // zero parts with an infinite weight are NaN where the fp32 product need
-    // not be; an output that came out NaN is formed again in plain fp32
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int32_t r = wv * WR + 16 * i + 4 * lg + e, t = 16 * j + l16;
-                if (acc[i][j][e] != acc[i][j][e] && r < wrows_here && t < rows_here) {
-                    const uint16_t* wp = reinterpret_cast<const uint16_t*>(w + static_cast<size_t>(n0 + r) * rbytes);
-                    const float* xp = x + static_cast<size_t>(t0 + t) * k;
-                    float sum = 0.0f;
-                    for (int32_t q = kb; q < ke; ++q)
-                        sum += __builtin_bit_cast(float, static_cast<uint32_t>(wp[q]) << 16) * xp[q];
-                    acc[i][j][e] = sum;
-                }
-            }
-
     // the tile through LDS as [token][row], then whole token rows out
     __syncthreads();
     float* ost = reinterpret_cast<float*>(smem);
+    int nan_out = 0;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NT; ++j) {
             *reinterpret_cast<floatx4*>(&ost[(16 * j + l16) * OLD + wv * WR + 16 * i + 4 * lg]) = acc[i][j];
-    __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) nan_out |= acc[i][j][e] != acc[i][j][e];
+        }
+    if (__syncthreads_or(nan_out)) {
+        // A NaN output may be one of the parts alone (those of an infinite x, a
+        // zero part times an infinite weight): formed again in plain fp32, a
+        // wave per output.  A token or weight row found to hold a NaN
+        // has NaN outputs only, and costs each wave one such sum.  (14336 ->
+        // 4096 at B = 64, 50 us: one token infinite 117, all NaN 89, all infinite
+        // 2410; with a lane per output 835, 7590 and 7580.)
+        constexpr int CH = BN / 64;  // chunks of 64 rows; a wave takes every 8 / CH-th token of one chunk
+        const int ch = wv % CH, c = 64 * ch + lane;
+        uint64_t nan_rows = 0;
+        for (int t = wv / CH; t < rows_here; t += 8 / CH) {
+            const float v = ost[t * OLD + c];
+            uint64_t todo = __ballot(v != v && c < wrows_here) & ~nan_rows;
+            while (todo) {
+                const int r = 64 * ch + __builtin_ctzll(todo);
+                const uint8_t* wp = w + static_cast<size_t>(n0 + r) * rbytes;
+                const float* xp = x + static_cast<size_t>(t0 + t) * k;
+                float sum = 0.0f;
+                bool wn = false, xn = false;
+                for (int32_t q = kb + 8 * lane; q < ke; q += 512) {
+                    const uint4 wq = *reinterpret_cast<const uint4*>(wp + 2 * static_cast<size_t>(q));
+                    const float4 xa = *reinterpret_cast<const float4*>(xp + q), xb = *reinterpret_cast<const float4*>(xp + q + 4);
+                    const uint32_t wd[4] = {wq.x, wq.y, wq.z, wq.w};
+                    const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float wf = __builtin_bit_cast(float, (e & 1) == 0 ? wd[e >> 1] << 16 : wd[e >> 1] & 0xffff0000u);
+                        sum += wf * xv[e];
+                        wn = wn || wf != wf;
+                        xn = xn || xv[e] != xv[e];
+                    }
+                }
+                sum = wave_sum(sum);
+                if (lane == 0) ost[t * OLD + r] = sum;
+                if (__any(wn)) nan_rows |= todo & -todo;
+                todo &= todo - 1;
+                if (__any(xn)) break;
+            }
+        }
+        __syncthreads();
+    }
     float* dst = gridDim.z > 1 ? part + static_cast<size_t>(bz) * b * n : y;
     if ((n & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
         constexpr int LPT = BN / 4, TPI = 512 / LPT;

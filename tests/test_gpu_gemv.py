@@ -318,10 +318,11 @@ def test_matbatch_bf16_exact_parts(lib, k, n, b):
     assert rel_l2(y, x.astype(np.float64) @ wf.T) < 3e-7  # measured 0.7e-7 to 1.3e-7
 
 
-def test_matbatch_bf16_infinite_and_nan(lib):
+@pytest.mark.parametrize("k,n,b", [(2048, 1000, 40), (1032, 16500, 258), (4096, 700, 16)])
+def test_matbatch_bf16_infinite_and_nan(lib, k, n, b):
     """Infinite and NaN activations and weights give what the fp32 products
-    give: a zero lower part times an infinite weight is no NaN."""
-    k, n, b = 2048, 1000, 40
+    give (a zero lower part times an infinite weight is no NaN), in their own
+    outputs only: K split, not split, and one 16-token tile."""
     w = synth.make_weights(BF16, n, k, seed=8500)
     x = synth.make_activations(b, k, seed=8501).reshape(b, k).copy()
     x[0, 5] = np.inf
@@ -331,20 +332,32 @@ def test_matbatch_bf16_infinite_and_nan(lib):
     # near the top of fp32 in one place: |w| < 0.2 there, so no sum in any order
     # leaves fp32 (a whole row of such values overflows in some orders only)
     x[4, 3] = np.float32(3.4e38)
+    x[5, 700] = np.array(0x7F800001, np.uint32).view(np.float32)  # a NaN whose upper half is infinity's
+    x[6] = np.inf
+    x[7] = np.nan
+    x[8, 6], x[8, 8] = np.inf, -np.inf
     wu = w.view(np.uint16).reshape(n, k)
     wu[10, 11] = 0x7F80  # +inf
     wu[11, 12] = 0xFF80  # -inf
+    wu[300, 13] = 0x7FC0  # NaN
+    wu[301, 14], wu[301, 15] = 0x7F80, 0xFF80
+    wu[n - 1] = 0x7F80
     y = np.zeros((b, n), np.float32)
     lib.gncx_xfold_universal_matbatch(ptr(w), 0, BF16, ptr(x), b, k, n, ptr(y), None)
     gncx.check(lib)
-    wf = (wu.astype(np.uint32) << 16).view(np.float32)
     with np.errstate(all="ignore"):
-        want = np.stack([(x[t][None, :] * wf).astype(np.float64).sum(1) for t in range(b)])
+        wf = (wu.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        xf = x.astype(np.float64)
+        want = xf @ wf.T
+        bound = (3 * 4 + 8 + k // 1024 + 256) * 2.0 ** -23 * (np.abs(xf) @ np.abs(wf).T) + 1e-37  # as above
     assert np.array_equal(np.isnan(y), np.isnan(want))
     big = np.abs(want) > 3e38
     assert np.array_equal(np.sign(y[big]), np.sign(want[big]))
     inf = np.isinf(want)
     assert np.array_equal(y[inf], want[inf].astype(np.float32))
+    finite = np.isfinite(want)
+    assert np.mean(finite) > 0.5  # (16 tokens: 9 of them with special values)
+    assert np.all(np.abs(y[finite] - want[finite]) <= bound[finite])
 
 
 # The streamed kernel's token tiles (16, 32, 64, 128) at their edges, Q8_0 and
