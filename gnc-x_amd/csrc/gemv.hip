@@ -655,13 +655,13 @@ bool try_band_ext_type(int32_t type, const BandMats& m, const float* x, int32_t 
 // ONE for 16-wave groups with at least kOneMinRowWaves row-waves, and for
 // Q4_K / Q8_0 rows split into three or more K-slices (Q4_K 12288 x 4096:
 // 8.2 vs 8.8 us under TWO; Q8_0 14336 x 4096: 14.3 vs 15.5 us); TWO otherwise
-// (BF16: TWO; the wide slots read zeros past the row only through its buffers)
+// (wide BF16 slots: TWO, whose buffers alone read zeros past the row)
 template <int TYPE, int THREADS>
 bool try_band(const BandMats& m, const float* x, int32_t k, int32_t n, hipStream_t stream) {
     const int32_t nwk = (Slot<TYPE>::slots(k) + 63) / 64;
     const bool one = nwk >= 1 && ((THREADS / 64) / nwk >= kOneMinRowWaves ||
                                   (nwk >= 3 && (TYPE == kQ4_K || TYPE == kQ8_0)));
-    if constexpr (THREADS == 1024 && !is_bf16(TYPE))
+    if constexpr (THREADS == 1024 && TYPE != kBF16Wide)
         if (one && try_band_sched<TYPE, THREADS, kSchedOne>(m, x, k, n, stream)) return true;
     return try_band_sched<TYPE, THREADS, kSchedTwo>(m, x, k, n, stream);
 }
@@ -693,13 +693,23 @@ hipError_t launch_band_type(int32_t type, const BandMats& m, const float* x, int
     case kQ4_K: return launch_band<kQ4_K>(m, x, k, n, stream, used);
     case kQ6_K: return launch_band<kQ6_K>(m, x, k, n, stream, used);
     case kBF16: {
-        // 16-byte slots where a row's K-slices fill the 16 waves twice (K from
-        // 3585 to 4096), else two pieces per lane.  Narrow / wide: 4096 x 4096
-        // 7.55 / 7.75 us, 4096 x 100000 123 / 131; 1024 x 50000 22.6 / 18.0,
-        // 5000 x 7000 15.2 / 12.7, 8192 x 8192 24.3 / 23.4; past K = 8192 the
-        // narrow slots do not fit 16 waves (gemv_kernel): 14336 x 4096 31.4 /
-        // 21.3, 16384 x 5000 53.6 / 29.2
-        const bool narrow = (Slot<kBF16>::slots(k) + 63) / 64 == 8;
+        // Two pieces per lane (wide slots) or one (narrow).  Wide slots halve a
+        // row's waves, which pays while the waves left have rows to take.
+        // Narrow / wide, us a call of a replayed graph:
+        //   1 narrow slice (K <= 512), few rows: 256 x 512 2.87 / 2.81, but
+        //     256 x 4096 3.32 / 3.38, 64 x 14336 4.37 / 4.68 (schedule ONE)
+        //   2: 1024 x 512 3.34 / 3.21, 1024 x 8192 6.53 / 6.02
+        //   3 to 16 (K <= 8192), up to 64 KB of weights per work-group: 2048 x
+        //     4096 5.70 / 6.06, 8192 x 1024 5.75 / 6.17; above: 2048 x 8192 8.22 /
+        //     8.15, 3072 x 4096 7.68 / 7.11, 5120 x 4096 11.6 / 9.7, 8192 x 4096
+        //     13.9 / 13.2
+        //   8 (K from 3585 to 4096) fill the 16 waves twice: 4096 x 4096 7.55 /
+        //     7.75, 4096 x 100000 123 / 131
+        //   past 16 the narrow slots do not fit 16 waves (gemv_kernel): 14336 x
+        //     4096 30.7 / 21.3
+        const int32_t slices = (Slot<kBF16>::slots(k) + 63) / 64;
+        const size_t per_group = row_bytes(kBF16, k) * static_cast<size_t>(n) / (n < kBandGroups ? n : kBandGroups);
+        const bool narrow = slices == 8 || (per_group <= 65536 && (slices == 1 ? n >= 4096 : slices >= 3 && slices <= 16));
         return narrow ? launch_band<kBF16>(m, x, k, n, stream, used) : launch_band<kBF16Wide>(m, x, k, n, stream, used);
     }
     default: used = false; return hipErrorInvalidValue;

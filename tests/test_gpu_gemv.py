@@ -91,11 +91,15 @@ def test_matvec_parity(lib, oracle, t, k, n):
     assert err < TOL
 
 
-# BF16 rows in slots of two 8-weight pieces (every K but 3585 to 4096): one
-# piece, 64 pieces, one more, a last slice with and without second pieces, the
-# longest row that fits 16 waves and one past it, and rows of the narrow slots
-@pytest.mark.parametrize("k,n", [(8, 5), (512, 300), (520, 257), (1024, 1000), (1544, 33), (2040, 700), (3584, 65),
-                                 (3592, 300), (4096, 1030), (4104, 300), (16384, 70), (16392, 40)])
+# BF16 rows in wide slots (two 8-weight pieces) and narrow ones (one), each at
+# the edges of the sizes that take it: a row of one piece, 64 pieces, one more, a
+# last slice with and without second pieces, the longest row of 16 waves and one
+# past it (wide: (512, 300) to (16384, 70)); narrow: K <= 512 from 4096 rows,
+# more than two slices up to 64 KB of weights per work-group, K from 3585 to 4096
+@pytest.mark.parametrize("k,n", [(8, 5), (512, 300), (520, 257), (1024, 1000), (2040, 8300), (3584, 4000),
+                                 (4104, 3000), (8192, 1030), (16384, 70), (16392, 40),
+                                 (8, 4096), (512, 4099), (1032, 515), (1544, 33), (2040, 700), (3584, 65),
+                                 (3592, 300), (4096, 1030), (4104, 300), (8192, 1024)])
 def test_matvec_bf16_slots(lib, k, n):
     w = synth.make_weights(BF16, n, k, seed=1100 + k + n)
     x = synth.make_activations(1, k, seed=2100 + k + n)
