@@ -603,15 +603,18 @@ __global__ __launch_bounds__(kThreads) void attn_mq_kernel(AttnParams p) {
 // Causal prefill: B query tokens at positions pos0 .. pos0 + B - 1, each with
 // the semantics of one decode step at its position (write its K/V row, then
 // attend over its window).  Two launches:
-//   attn_prefill_prologue_kernel: per token, the heads-RMSNorm + RoPE
-//     prologue of q and k in LDS (the decode prologue's arithmetic, with the
-//     token's own host-made cos/sin row), q written back, K/V rows stored;
+//   attn_prefill_prologue_kernel: the heads-RMSNorm + RoPE prologue of q and
+//     k, 16 heads of a token per work-group (the decode prologue's arithmetic,
+//     with the token's own host-made cos/sin row), q and k written back, K/V
+//     rows stored;
 //   attn_prefill_kernel (head_dim 128, G = n_heads / n_kv dividing 32): a
 //     work-group owns 128 query rows, 128 / G tokens x the G heads of one KV
 //     head, and walks the block's whole key range in 32-key sub-chunks with
 //     S^T = K Q^T, online softmax and O += P V (fp16 matrix cores, fp16-pair
 //     operands), masking each row to its own causal window, and writes
-//     out = O / (l + 1e-12) directly (no split, no merge).
+//     out = O / (l + 1e-12) directly;
+//   with a key-split plan a work-group walks one part of a long block's range,
+//     and attn_prefill_merge_kernel, a third launch, combines the parts.
 struct PrefillParams {
     float* q;             // [B][n_heads * HD], prologue result in place
     float* k;             // [B][n_kv * HD], prologue result in place
@@ -639,8 +642,8 @@ struct PrefillParams {
 // head_inv_rms does for one head (the same fp32 lane sums, added in double),
 // but for 16 heads at once in one wave: those chains of 32 dependent adds, ten
 // heads after one another per wave, were what a token waited for.  KV heads
-// also store their K and V rows.  2048 tokens x 40 heads: 33 us -> TIMEB;
-// -> 21.0 us (104 MB), 300 tokens 18.6 -> 5.7 us.
+// also store their K and V rows.  2048 tokens x 40 heads (104 MB): 33 -> 21.0
+// us, 300 tokens 18.6 -> 5.7 us.
 constexpr int kProHeads = 16;
 __global__ __launch_bounds__(kThreads) void attn_prefill_prologue_kernel(PrefillParams p) {
 #pragma clang fp contract(off)
@@ -801,7 +804,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_prefill_kernel(PrefillParams
     const int nq = min(TQ, p.batch - q0);
     const int hi_block = p.pos0 + q0 + nq - 1;
     const int lo_block = p.sw > 0 ? max(0, p.pos0 + q0 - p.sw + 1) : 0;
-    // this work-group's keys: the block's range, or one half of it
+    // this work-group's keys: the block's range, or one part of it
     const int lo_first = p.plan ? reinterpret_cast<const int4*>(p.plan)[blockIdx.y].z : lo_block;
     const int hi_last = p.plan ? reinterpret_cast<const int4*>(p.plan)[blockIdx.y].w : hi_block;
     const size_t kv_dim = static_cast<size_t>(p.n_kv) * HD;
@@ -967,7 +970,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_prefill_kernel(PrefillParams
         __syncthreads();  // every wave is done with this sub-chunk's K / V fragments
     }
     if (slot >= 0) {
-        // half of a split block: the unnormalised O and the row's (max, sum)
+        // a part of a split block: the unnormalised O and the row's (max, sum)
         // for attn_prefill_merge_kernel
         const size_t base = (static_cast<size_t>(slot) * p.n_kv + hk) * kPfRows;
         if (g == 0)
@@ -1326,7 +1329,10 @@ bool attention_prefill_supported(int32_t n_heads, int32_t n_kv_heads, int32_t he
     if (head_dim != 128 || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads != 0) return false;
     const int32_t G = n_heads / n_kv_heads;
     if (G > 32 || 32 % G != 0) return false;
-    return sizeof(float) * static_cast<size_t>(n_heads + n_kv_heads) * head_dim <= kLdsBudget;
+    // up to 128 heads in all.  Nothing in the kernels needs that, but they hold V
+    // as fp16 pairs (|v| < 65504) and the per-token steps do not: the route is
+    // not widened to shapes that it has not served
+    return n_heads + n_kv_heads <= 128;
 }
 
 size_t attention_prefill_part_floats(int32_t part_slots, int32_t n_kv_heads) {
@@ -1337,14 +1343,14 @@ constexpr size_t kPfPartMax = size_t{128} << 20;
 // The key-split plan of a prefill call.  A block's work is its number of
 // 32-key sub-chunks, and two work-groups share a CU, so the kernel's time is
 // about the larger of its longest work-group and the total work over the
-// resident work-groups.  Blocks longer than a third of the longest (and than
-// 8 sub-chunks; less where the grid is short, below) are cut into parts of their key range of at most that
-// length, each a work-group, whose partial results attn_prefill_merge_kernel
-// combines; grid rows are ordered longest first.  (2048 tokens, 32/8 heads:
-// kernel + merge 200 us per layer unsplit; halves 163 + 12, thirds best,
-// quarters 149 + 21: the partials' traffic grows with the parts.)  Up to 8
-// sub-chunks in the longest block there is nothing worth a second launch: no
-// plan.
+// resident work-groups.  Blocks longer than a third of the longest (and than 8
+// sub-chunks; less where the grid is short, below) are cut into parts of their
+// key range of at most that length, each a work-group, whose partial results
+// attn_prefill_merge_kernel combines; grid rows are ordered longest first.
+// (2048 tokens, 32/8 heads: kernel + merge 200 us per layer unsplit; halves 163
+// + 12, thirds best, quarters 149 + 21: the partials' traffic grows with the
+// parts.)  Up to 8 sub-chunks in the longest block there is nothing worth a
+// second launch: no plan.
 // Table: n_items rows of (block, slot, first key, last key), slot -1 for a
 // whole block, else its part's index in the partial buffers; then per split
 // block (block, first slot, parts).

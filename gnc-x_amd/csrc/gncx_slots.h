@@ -97,29 +97,6 @@ struct BufRow {
     __device__ __forceinline__ uint32_t sh(int32_t o) const { return (delta + static_cast<uint32_t>(o)) & 3u; }
 };
 
-// Rows of a tile read through one wave-uniform resource over the tile's rows
-// (4-aligned base); each lane adds the byte offset of its own row.  A lane
-// with no row uses an offset past the resource and reads zeros.
-struct TileRow {
-    __amdgpu_buffer_rsrc_t r;
-    int32_t base;
-    __device__ __forceinline__ u32x4 ld16(int32_t o) const {
-        return __builtin_amdgcn_raw_buffer_load_b128(r, base + o, 0, 0);
-    }
-    __device__ __forceinline__ u32x4a4 ld16a4(int32_t o) const {
-        return __builtin_amdgcn_raw_buffer_load_b128(r, base + o, 0, 0);
-    }
-    __device__ __forceinline__ u32x2a4 ld8a4(int32_t o) const {
-        return __builtin_amdgcn_raw_buffer_load_b64(r, base + o, 0, 0);
-    }
-    __device__ __forceinline__ uint32_t ldu16(int32_t o) const {
-        return __builtin_amdgcn_raw_buffer_load_b16(r, base + o, 0, 0);
-    }
-    __device__ __forceinline__ u32x4 ld16u(int32_t o) const { return __builtin_amdgcn_raw_buffer_load_b128(r, base + o, 0, 0); }
-    __device__ __forceinline__ u32x2 ld8u(int32_t o) const { return __builtin_amdgcn_raw_buffer_load_b64(r, base + o, 0, 0); }
-    __device__ __forceinline__ uint32_t sh(int32_t o) const { return static_cast<uint32_t>(base + o) & 3u; }
-};
-
 // raw 16-byte field at a 2-aligned row offset o: the dword-aligned dwordx4 at
 // o - sh and the 2 bytes at o + 14 (see ld16_a2); sh = field address mod 4 is
 // kept by the caller (all fields of one block share it) and the field is

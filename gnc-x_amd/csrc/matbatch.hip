@@ -61,29 +61,7 @@ __global__ __launch_bounds__(kThreads) void matbatch_rowtok_kernel(const uint8_t
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2 __attribute__((ext_vector_type(2)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// act_q_kernel<U> holds U float4 of x per thread in registers from the
-// max pass to the quantising pass (rows up to 4 kThreads U values): the
-// loads of a row are issued together, and a longer row reads its tail again.
-// U = 4 covers 4096-wide rows; wider rows take U = 16, or, for the SwiGLU rows
-// of the down projection up to 12288 wide, 1024 threads (NT) with U = 3, which
-// keeps more of a row's loads in flight (47.9 -> 45.1 us at 2048 x 12288).
-
-// The reference's per-32 quantisation of row blockIdx.x of x (cpp:955-995):
-// the quantised values q as fp16 (integers of at most 127, exact), row-major
-// [B x K], and each 32-block's d / s as fp32 [B x K / 32], s the power of two
-// above the row's largest |x| (stored in rscale; the product's epilogue
-// multiplies it back, exactly).  Within each 8 values the order is 0 2 1 3 4
-// 6 5 7, the product kernel's operand order.  With pq given (K a multiple of
-// 256), also each 32-block's sum of the quantised activations, P = (sum q) *
-// d / s, as an fp16 pair: per token row and 256-value super-block, 8 hi then
-// 8 lo values (the Q4_K kernel's min term, cpp:1177-1178); the scale keeps P
-// within fp16's range for activations of 1e5 and more (SwiGLU outputs).
-// One work-group per row: the row maximum first, then 8 lanes per 32-block,
-// 4 values per lane.
-// With SW the row is the SwiGLU of two rows, x the gates and up the ups
-// (the values gncx_swiglu_activation writes), formed as they are read.
 // One task's outputs (4 values of row `row`, task t of k / 4, at the
 // row's 1 / s = inv): q as fp16, the block's d / s from its first lane and,
 // with pq, the block's P pair.  Whole 8-lane groups call it together.
@@ -115,6 +93,26 @@ __device__ __forceinline__ void emit_q(const float4 v, int32_t t, int32_t row, i
     }
 }
 
+// The reference's per-32 quantisation of row blockIdx.x of x (cpp:955-995):
+// the quantised values q as fp16 (integers of at most 127, exact), row-major
+// [B x K], and each 32-block's d / s as fp32 [B x K / 32], s the power of two
+// above the row's largest |x| (stored in rscale; the product's epilogue
+// multiplies it back, exactly).  Within each 8 values the order is 0 2 1 3 4
+// 6 5 7, the product kernel's operand order.  With pq given (K a multiple of
+// 256), also each 32-block's sum of the quantised activations, P = (sum q) *
+// d / s, as an fp16 pair: per token row and 256-value super-block, 8 hi then
+// 8 lo values (the Q4_K kernel's min term, cpp:1177-1178); the scale keeps P
+// within fp16's range for activations of 1e5 and more (SwiGLU outputs).
+// One work-group per row: the row maximum first, then 8 lanes per 32-block,
+// 4 values per lane.
+// With SW the row is the SwiGLU of two rows, x the gates and up the ups
+// (the values gncx_swiglu_activation writes), formed as they are read.
+// act_q_kernel<U> holds U float4 of x per thread in registers from the
+// max pass to the quantising pass (rows up to 4 kThreads U values): the
+// loads of a row are issued together, and a longer row reads its tail again.
+// U = 4 covers 4096-wide rows; wider rows take U = 16, or, for the SwiGLU rows
+// of the down projection up to 12288 wide, 1024 threads (NT) with U = 3, which
+// keeps more of a row's loads in flight (47.9 -> 45.1 us at 2048 x 12288).
 template <int U, bool SW = false, int NT = kThreads>
 __global__ __launch_bounds__(NT) void act_q_kernel(const float* __restrict x, int32_t k, uint2* __restrict xq,
                                                    float* __restrict rscale, _Float16* __restrict pq,
@@ -193,8 +191,9 @@ void launch_act_q(const float* x, int32_t b, int32_t k, const QsBufs& q, hipStre
             hipLaunchKernelGGL((act_q_kernel<16, true>), dim3(b), dim3(kThreads), 0, stream, x, k, o, q.rscale, q.pq,
                                up, q.dxs);
     } else if (b <= 512 && k > 2048 && k <= 4 * 4 * 1024) {
-        // few long rows: 16 waves each (4096 x 1438 at K = 5504, B = 113: 36.2 ->
-        // 30.4 us with the paired stores below; rows up to 2048 gain nothing)
+        // few long rows: 16 waves each (whole calls, Q6_K 14336 -> 4096 at B = 64
+        // 41.7 -> 40.3 us, Q8_0 5504 -> 1438 at B = 113 30.6 -> 30.0; at B = 512
+        // and for rows up to 2048 no gain)
         if (k <= 4 * 1024)
             hipLaunchKernelGGL((act_q_kernel<1, false, 1024>), dim3(b), dim3(1024), 0, stream, x, k, o, q.rscale, q.pq,
                                nullptr, q.dxs);
@@ -326,7 +325,7 @@ __device__ __forceinline__ void step_barrier() {
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
-// The matrices of one Q4_K launch (one activation batch, the same K): x-tiles
+// The matrices of one launch (one activation batch, the same K): x-tiles
 // [tile0[i], tile0[i + 1]) are matrix i, n[i] rows, output y[i] [b x n[i]].
 // A work-group picks its matrix with scalar compares and selects over the
 // kernel arguments.  With split K the partials of range z are one [b x ntot]
@@ -390,7 +389,8 @@ struct RedMats {
 //
 // The activations (q as fp16, d_x / s per block and, for the min term, P
 // pairs) stream through three LDS stages, one super-block each, filled by
-// direct-to-LDS loads two super-blocks ahead; one barrier per super-block.
+// direct-to-LDS loads two super-blocks ahead (128 tokens: two stages, which
+// fill the LDS, one ahead); one barrier per super-block.
 // With gridDim.z > 1 the result is a split-K partial.  It leaves through LDS,
 // so that each store instruction writes one token's contiguous row range.
 constexpr int kQsRows = 256;  // weight rows per work-group
@@ -755,18 +755,15 @@ __global__ __launch_bounds__(512, 1) void matbatch_qs_stream_kernel(
     const int32_t rows_here = min(BM, b - t0), wrows_here = min(BN, n - n0);
 
     // this lane's weight rows, 32 wv + 16 f + l % 16; rows past N and
-    // super-blocks past the range read zeros (offsets past the resource,
-    // whose base is the dword at or below the first row)
+    // super-blocks past the range read zeros (offsets past the resource)
     using W = QsW<TYPE, kQsWide<TYPE, TF>>;
     using H = QsH<TYPE>;
     constexpr int32_t kWB = TYPE == kQ6_K ? 210 : TYPE == kQ8_0 ? 272 : 144;  // bytes of a super-block
-    const uint8_t* wt = w + static_cast<size_t>(n0) * rbytes;
-    const int32_t delta = TYPE == kQ4_K ? 0 : static_cast<int32_t>(reinterpret_cast<uintptr_t>(wt) & 3u);
-    const __amdgpu_buffer_rsrc_t wrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wt - delta), static_cast<short>(0),
-                                          wrows_here * static_cast<int32_t>(rbytes) + delta, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(w + static_cast<size_t>(n0) * rbytes), static_cast<short>(0),
+        wrows_here * static_cast<int32_t>(rbytes), 0x00020000);
     auto row_at = [&](int32_t row) {
-        return row < wrows_here ? row * static_cast<int32_t>(rbytes) + delta + kb / 256 * kWB : kMfOob / 2;
+        return row < wrows_here ? row * static_cast<int32_t>(rbytes) + kb / 256 * kWB : kMfOob / 2;
     };
     const int32_t wbase[RF] = {row_at(32 * wv + l16), row_at(32 * wv + 16 + l16)};
     const int32_t hbase = row_at(32 * wv + (lane & 31));

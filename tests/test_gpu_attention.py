@@ -357,7 +357,7 @@ PREFILL_CASES = [
     (16, 16, 128, 0, 40, 0),
     (8, 2, 64, 2, 10, 0),
     # key ranges of more than 8 sub-chunks of 32 keys: the longer blocks are
-    # cut into up to three work-groups whose parts a merge kernel combines --
+    # cut into up to eight work-groups whose parts a merge kernel combines --
     # a fresh prompt, a cache prefix (every block cut), a sliding window, MQA,
     # and one head per KV head (128-token blocks)
     (32, 8, 128, 0, 600, 0),

@@ -259,29 +259,28 @@ def test_matvec_device_pointers(lib, oracle):
 
 
 # quantised types run on the fp16 matrix cores with exact integer operands; cases
-# cover every tile size the launcher picks, split K, ragged B and N, and K with
-# an odd number of 32-wide steps (k % 64 == 32)
+# cover split and whole K, ragged B and N, K with an odd number of 32-value
+# blocks, and every token tile (16, 32, 64, 128; test_matbatch_stream_steady_state
+# has each type on each)
 MATBATCH_CASES = [
     (Q4_K, 4096, 512, 64), (Q6_K, 14336, 256, 16), (Q4_0, 4096, 300, 5), (Q8_0, 2048, 200, 9), (Q4_K, 512, 96, 1),
     (BF16, 1024, 64, 4), (Q4_K, 4096, 1024, 256), (Q6_K, 2048, 4160, 100), (Q4_0, 96, 130, 70),
     (Q8_0, 2080, 333, 33),
     (Q4_K, 256, 16384, 300),
     (Q4_K, 256, 8192, 500), (Q6_K, 256, 16384, 128), (Q4_K, 256, 16384, 512), (Q6_K, 512, 8192, 520),
-    # the 256-token tiles of 8 waves (256 x 128 and 256 x 64), ragged B and N
+    # one and two super-blocks, a token or more past whole tiles
     (Q6_K, 256, 24576, 260), (Q4_K, 256, 8192, 300), (Q8_0, 512, 6000, 257),
-    # the 8-wave tiles with K split (Q4_K 64 x 256 up to 128 tokens, 128 x 256
-    # above; 256 x 128 from 129 tokens for the other types), ragged B and N
+    # K split, ragged B and N
     (Q4_K, 2048, 1000, 100), (Q4_K, 4096, 3000, 65), (Q6_K, 4096, 1000, 300), (Q8_0, 2080, 700, 400),
     (Q4_K, 4096, 3000, 200), (Q4_K, 2048, 700, 33),
-    # 128 x 128 tiles of 4 waves with K split (65 to 128 tokens, types other than Q4_K)
+    # 65 to 128 tokens
     (Q8_0, 1024, 640, 128), (Q6_K, 14336, 512, 77),
     # Q4_K at small B: one super-block, K of 3, 5 and 48 super-blocks, ragged B and N
     (Q4_K, 256, 100, 17), (Q4_K, 768, 50, 64), (Q4_K, 1280, 33, 2), (Q4_K, 12288, 200, 48),
-    # Q4_K one-product kernel (B >= 1024, whole K): ragged B and N, one and 8 super-blocks
+    # more than 1024 tokens
     (Q4_K, 2048, 1000, 1100), (Q4_K, 256, 520, 1030),
-    # Q4_K short batches (weights streamed through registers, up to 64 tokens):
-    # one and two token tiles, ragged N, K ranges of 1 to 8 super-blocks (the
-    # three register sets in turn, ranges of unequal length), one token
+    # Q4_K short batches: ragged N, K ranges of one super-block and more, whole
+    # K, one token
     (Q4_K, 12288, 1030, 64), (Q4_K, 20480, 300, 1), (Q4_K, 4096, 777, 40), (Q4_K, 2304, 4100, 63),
     (Q4_K, 4096, 16384, 32), (Q4_K, 2048, 24576, 50), (Q4_K, 3072, 40000, 20), (Q4_K, 1792, 40000, 9),
     (Q4_K, 4096, 6144, 64),
@@ -433,12 +432,13 @@ def test_matbatch_split_reduce(lib, oracle, k, n, b):
     assert rel_l2(y, want) < 5e-7
 
 
-# Q6_K scales beyond +-64 (real quantisers use the whole int8 range): then
-# sc (q - 32) can exceed 2048 and the 256-token tiles add the third product in
-# the steps that hold such a scale.  All rows large, none, and one row in
-# 37 large (single steps of a tile), with K split (k=2048, b=200) and unsplit.
+# Q6_K scales over the whole int8 range (real quantisers use it): sc (q - 32)
+# then needs 13 bits, and its two products, sc (l - 16) and 16 sc (u - 1), must
+# each be exact.  All rows, and one row in 37; K split (the first four) and whole
+# with 4 and 5 super-blocks (64 and 128 tokens).
 @pytest.mark.parametrize("mode", ["all", "sparse"])
-@pytest.mark.parametrize("k,n,b", [(2048, 512, 200), (1024, 3000, 300), (4096, 600, 64), (768, 300, 7)])
+@pytest.mark.parametrize("k,n,b", [(2048, 512, 200), (1024, 3000, 300), (4096, 600, 64), (768, 300, 7),
+                                   (1024, 40000, 50), (1280, 20000, 300)])
 def test_matbatch_q6k_large_scales(lib, oracle, mode, k, n, b):
     w = synth.make_weights(Q6_K, n, k, seed=8100 + k + n).reshape(n, k // 256, 210)
     rng = np.random.default_rng(8200 + b)
@@ -460,8 +460,8 @@ def test_matbatch_q6k_large_scales(lib, oracle, mode, k, n, b):
 
 # gncx_hip_swiglu_matbatch: the SwiGLU formed in the activation pass, bit for
 # bit the values of gncx_swiglu_activation followed by matbatch; K past the
-# quantiser's registers (20480), the one-product Q4_K kernel (B = 1024) and
-# BF16 weights (the rows formed first).
+# quantiser's registers (20480), more than 1000 tokens and BF16 weights (the rows
+# formed first).
 @pytest.mark.parametrize("t,k,n,b", [(Q4_K, 4096, 512, 64), (Q4_K, 12288, 256, 300), (Q4_K, 20480, 128, 7),
                                      (Q4_K, 12288, 256, 1024), (Q6_K, 2048, 300, 200), (Q8_0, 1024, 96, 33),
                                      (BF16, 512, 64, 5)])
@@ -485,7 +485,7 @@ def test_swiglu_matbatch_equals_two_calls(lib, t, k, n, b):
 
 # The prefill workloads at their own shapes: Q4_K 4096x4096 (Q/O) and
 # 4096 -> 14336 (gate/up), Q6_K 14336 -> 4096 (down), at B = 64, 256 and 512,
-# plus ragged B past one 256-token tile and the B = 2048 prefill of the
+# plus ragged B between whole tiles and the B = 2048 prefill of the
 # Qwen3-8B-shaped model (4096 -> 12288 and 12288 -> 4096).
 CONFIG3_CASES = [(t, k, n, b) for (t, k, n) in [(Q4_K, 4096, 4096), (Q4_K, 4096, 14336), (Q6_K, 14336, 4096)]
                  for b in (64, 256, 512)] + [
@@ -510,9 +510,9 @@ def test_matbatch_prefill_shapes(lib, oracle, t, k, n, b):
 # Q/K/V- and gate/up-like groups through gncx_hip_matbatch_multi: the batch is
 # quantised once, and the matrices share one launch (and, with split K, one
 # reduce) when each is whole 256-row tiles of the plan for their summed rows
-# (B = 64 and 100: 64-token tiles, K in 8 ranges; B = 300 and 512:
-# 128-token tiles, K in 4 and 2 ranges; B = 2048: no split); otherwise one
-# call per matrix (1000 rows: not whole tiles).
+# (B = 64 and 100: 32-token tiles, K in 4 and 8 ranges; B = 300: 64-token tiles
+# and 4 ranges; B = 512 and 2048: no split); otherwise one call per matrix (1000
+# rows: not whole tiles).
 MULTI_CASES = [((4096, 1024, 1024), 4096, b) for b in (64, 512, 2048)] + [
     ((1536, 1536), 1024, 300), ((4096, 1000), 2048, 2048), ((256, 512, 256, 1024), 2048, 100)]
 
