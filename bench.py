@@ -284,7 +284,8 @@ PREFILL_SHAPES = {"q4k_4096x4096_b2048": (12, 4096, 4096), "q4k_4096x12288_b2048
 def matbatch_extras(pkg, lib, torch, steps=20):
     """Matbatch at B = 64 / 256 / 512 on the prefill shapes, and the B = 2048
     prefill matrices of the Qwen3-8B-shaped model.  GFLOP/s count 2 B K N
-    (the useful products); the kernel issues three fp16 MFMA products each."""
+    (the useful products); the kernel issues one fp16 MFMA product for each
+    (Q6_K: two)."""
     mb = {}
     for name, (tt, kk, nn) in MATBATCH_SHAPES.items():
         for bb in (64, 256, 512):

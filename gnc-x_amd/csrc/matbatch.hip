@@ -379,13 +379,15 @@ struct RedMats {
 // halves the weights' unpacking and loads per output.
 // Full calls at 4096 x 12288, B = 2048 / 512, before (32 x 32 tiles of 64
 // tokens; Q8_0 and Q4_0: both operands as fp16 pairs, three products) and
-// now: Q4_K 413 / 130 -> 310 / 105 us, Q6_K 665 / 213 -> 452 / 146, Q8_0 650 /
-// 200 -> 425 / 140, Q4_0 635 / 196 -> 417 / 136; 64-token tiles 382 / 128 (Q4_K).
-// Bound (counters, Q4_K at B = 2048): VALU issue 62% of the cycles (512 of 846
-// instructions per wave and super-block are the block scales), LDS 50%, matrix
-// cores 32%, at a clock of 2.08 GHz.  With work taken out in a copy, 335 us
-// became 245 without the activation reads from LDS, 209 without products,
-// 280 without the scales, 311 without the unpacking.
+// now: Q4_K 413 / 130 -> 310 / 100 us, Q6_K 665 / 213 -> 430 / 135, Q8_0 650 /
+// 200 -> 412 / 140, Q4_0 635 / 196 -> 405 / 139; 64-token tiles 382 / 128 (Q4_K).
+// Bound (counters, Q4_K at B = 2048): VALU issue 64% of the cycles (512 of 977
+// instructions per wave and super-block, products apart, are the block scales),
+// matrix cores 33%, address path 29%, LDS 26% without conflicts, at a clock of
+// 2.1 GHz: no unit alone, with two waves per SIMD.  With work taken out in a
+// copy (before the 16-byte loads), 335 us became 245 without the activation
+// reads from LDS, 209 without products, 280 without the scales, 311 without the
+// unpacking.
 //
 // The activations (q as fp16, d_x / s per block and, for the min term, P
 // pairs) stream through three LDS stages, one super-block each, filled by
