@@ -433,9 +433,9 @@ def test_matbatch_split_reduce(lib, oracle, k, n, b):
 
 
 # Q6_K scales over the whole int8 range (real quantisers use it): sc (q - 32)
-# then needs 13 bits, and its two products, sc (l - 16) and 16 sc (u - 1), must
-# each be exact.  All rows, and one row in 37; K split (the first four) and whole
-# with 4 and 5 super-blocks (64 and 128 tokens).
+# then needs more than the 11 bits of fp16, and its two products, sc (l - 16) and
+# 16 sc (u - 1), must each be exact.  All rows, and one row in 37; K split (the
+# first four) and whole with 4 and 5 super-blocks (64 and 128 tokens).
 @pytest.mark.parametrize("mode", ["all", "sparse"])
 @pytest.mark.parametrize("k,n,b", [(2048, 512, 200), (1024, 3000, 300), (4096, 600, 64), (768, 300, 7),
                                    (1024, 40000, 50), (1280, 20000, 300)])
